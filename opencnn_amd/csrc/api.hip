@@ -79,8 +79,9 @@ thread_local const char* t_last_kernel = "";
 thread_local int t_last_grid = 0;       // workgroups of this thread's last fused-kernel launch
 thread_local int t_last_flag_set = -1;  // its flag set: -1 none, kSyncSets = the caller's storage
 
-// ---- hand-scheduled assembly kernels (gen_wino_f32_asm.py), loaded from the embedded code object
-extern "C" const char opencnn_wino_f32_asm_hsaco[];
+// ---- hand-scheduled assembly kernels, loaded from the embedded code objects
+extern "C" const char opencnn_wino_f32_asm_hsaco[];        // gen_wino_f32_asm.py
+extern "C" const char opencnn_wino_f32_split_asm_hsaco[];  // gen_wino_f32_split_asm.py
 extern "C" const char opencnn_wino_h16_asm_hsaco[];  // gen_wino_h16_asm.py
 
 // Workspace of opencnn_conv_forward_static: the transformed filter of one call.  One copy per
@@ -112,10 +113,15 @@ struct CallerFlags {
   const unsigned* ptr = nullptr;
 };
 
+// The fp32 assembly kernels, [kw == 4][whole tiles, _ragged, _packed]: the same names in both code objects.
+constexpr const char* kF32Kernels[2][3] = {
+    {"wino_f32_asm_kw2", "wino_f32_asm_kw2_ragged", "wino_f32_asm_kw2_packed"},
+    {"wino_f32_asm_kw4", "wino_f32_asm_kw4_ragged", "wino_f32_asm_kw4_packed"}};
+
 struct DeviceState {
-  hipModule_t module = nullptr, module_h16 = nullptr;
-  hipFunction_t kw2 = nullptr, kw4 = nullptr, kw2_ragged = nullptr, kw4_ragged = nullptr;
-  hipFunction_t kw2_packed = nullptr, kw4_packed = nullptr;
+  hipModule_t module[2] = {nullptr, nullptr}, module_h16 = nullptr;
+  // fp32: [0] on the fp32 MFMA, [1] on bf16 pieces; [kw == 4][whole tiles, _ragged, _packed]
+  hipFunction_t f32[2][2][3] = {};
   hipFunction_t f16_kw4 = nullptr, bf16_kw4 = nullptr, f16_kw4_ragged = nullptr, bf16_kw4_ragged = nullptr;
   hipFunction_t f16_kw4_packed = nullptr, bf16_kw4_packed = nullptr;
   unsigned* split_sync = nullptr;  // device address of g_split_sync (all sets) on this device
@@ -144,13 +150,13 @@ int device_state(DeviceState** out) {
   std::lock_guard<std::mutex> lock(mu);
   DeviceState& k = per_device[dev];
   if (!k.ready) {
-    if ((e = hipModuleLoadData(&k.module, opencnn_wino_f32_asm_hsaco)) != hipSuccess) return (int)e;
-    if ((e = hipModuleGetFunction(&k.kw2, k.module, "wino_f32_asm_kw2")) != hipSuccess) return (int)e;
-    if ((e = hipModuleGetFunction(&k.kw4, k.module, "wino_f32_asm_kw4")) != hipSuccess) return (int)e;
-    if ((e = hipModuleGetFunction(&k.kw2_ragged, k.module, "wino_f32_asm_kw2_ragged")) != hipSuccess) return (int)e;
-    if ((e = hipModuleGetFunction(&k.kw4_ragged, k.module, "wino_f32_asm_kw4_ragged")) != hipSuccess) return (int)e;
-    if ((e = hipModuleGetFunction(&k.kw2_packed, k.module, "wino_f32_asm_kw2_packed")) != hipSuccess) return (int)e;
-    if ((e = hipModuleGetFunction(&k.kw4_packed, k.module, "wino_f32_asm_kw4_packed")) != hipSuccess) return (int)e;
+    const char* const images[2] = {opencnn_wino_f32_asm_hsaco, opencnn_wino_f32_split_asm_hsaco};
+    for (int m = 0; m < 2; ++m) {
+      if ((e = hipModuleLoadData(&k.module[m], images[m])) != hipSuccess) return (int)e;
+      for (int i = 0; i < 6; ++i)
+        if ((e = hipModuleGetFunction(&k.f32[m][i / 3][i % 3], k.module[m], kF32Kernels[i / 3][i % 3])) != hipSuccess)
+          return (int)e;
+    }
     if ((e = hipModuleLoadData(&k.module_h16, opencnn_wino_h16_asm_hsaco)) != hipSuccess) return (int)e;
     if ((e = hipModuleGetFunction(&k.f16_kw4, k.module_h16, "wino_f16_asm_kw4")) != hipSuccess) return (int)e;
     if ((e = hipModuleGetFunction(&k.bf16_kw4, k.module_h16, "wino_bf16_asm_kw4")) != hipSuccess) return (int)e;
@@ -563,7 +569,8 @@ struct AsmLaunch {
   hipFunction_t fn = nullptr;
   const char* name = "";
   int grid = 0;
-  size_t lds_bytes = 0;
+  unsigned threads = 256;   // per workgroup
+  size_t lds_bytes = 0;     // dynamic
   int chunks = 0;           // units per workgroup tile
   long long usw_bytes = 0;  // size of the transformed filter
   // The divisor that takes a workgroup tile index apart: the column blocks (filter-block major
@@ -686,7 +693,7 @@ int launch_asm_kernel(const opencnn::ConvArgs& a, const AsmLaunch& l, hipStream_
   size_t ka_size = sizeof(ka);
   void* extra[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, &ka, HIP_LAUNCH_PARAM_BUFFER_SIZE, &ka_size,
                    HIP_LAUNCH_PARAM_END};
-  const hipError_t e = hipModuleLaunchKernel(l.fn, (unsigned)grid, 1, 1, 256, 1, 1, (unsigned)l.lds_bytes,
+  const hipError_t e = hipModuleLaunchKernel(l.fn, (unsigned)grid, 1, 1, l.threads, 1, 1, (unsigned)l.lds_bytes,
                                              st, nullptr, extra);
   if (e == hipSuccess) {
     t_last_kernel = l.name;
@@ -779,27 +786,31 @@ int choose_range_weight(int tiles, int chunks, int ranges) {
   return best;
 }
 
+// Which of the two fp32 kernels: on bf16 pieces (six bf16 products per fp32 one, more than two and a half
+// times the matrix rate and the vector work next to it, but an output transform twice as long: its
+// workgroup exchanges 256 KB through LDS) from three 8-channel units per tile on.  Measured, fused
+// kernel in us, fp32 MFMA / pieces: C = 3, 64 x 224 x 224, K = 64 222 / 231; C = 16, 64 x 112 x 112, K = 64
+// 83.3 / 85.7; C = 24, 64 x 56 x 56, K = 96 58.0 / 54.0; C = 32, 32 x 28 x 28, K = 64 12.4 / 11.0; C = 64,
+// 64 x 56 x 56, K = 64 65.2 / 59.0; C = 512, 128 x 7 x 7, K = 512 128 / 103.
+bool split_into_pieces(int chunks) { return chunks >= 3; }
+
 int launch_asm(const opencnn::ConvArgs& a, int kw, int grid, bool ragged, bool packed, size_t lds_bytes,
                hipStream_t st, LaunchPlan* plan) {
   DeviceState* ak = nullptr;
   if (int e = device_state(&ak)) return e;
   AsmLaunch l;
-  if (packed) {
-    l.fn = kw == 4 ? ak->kw4_packed : ak->kw2_packed;
-    l.name = kw == 4 ? "wino_f32_asm_kw4_packed" : "wino_f32_asm_kw2_packed";
-  } else if (ragged) {
-    l.fn = kw == 4 ? ak->kw4_ragged : ak->kw2_ragged;
-    l.name = kw == 4 ? "wino_f32_asm_kw4_ragged" : "wino_f32_asm_kw2_ragged";
-  } else {
-    l.fn = kw == 4 ? ak->kw4 : ak->kw2;
-    l.name = kw == 4 ? "wino_f32_asm_kw4" : "wino_f32_asm_kw2";
-  }
+  const int form = packed ? 2 : (ragged ? 1 : 0);
+  l.chunks = (a.C + 7) / 8;
+  const bool pieces = split_into_pieces(l.chunks);
+  l.fn = ak->f32[pieces][kw == 4][form];
+  l.name = kF32Kernels[kw == 4][form];
   l.packed = packed;
   l.grid = grid;
-  l.lds_bytes = lds_bytes;
-  l.chunks = (a.C + 7) / 8;
+  l.threads = pieces ? 512 : 256;
+  l.lds_bytes = pieces ? 0 : lds_bytes;  // (160 KB in its kernel descriptor)
   l.usw_bytes = padded_c(a.C) * 16 * padded_k(a.K) * 4;
-  l.tile_split = a.colblocks;
+  // (on pieces, kw 4: the column blocks of both filter blocks of a pair)
+  l.tile_split = pieces && kw == 4 ? 2 * a.colblocks : a.colblocks;
   l.c_real_or_mode = a.C;
   // Ranges of the balanced split that are at least a tile long may be cut on a weighted line.
   if (grid < a.nblocks && a.sync != nullptr)
@@ -1148,10 +1159,21 @@ int launch_on_flag_set(opencnn::ConvArgs& a, const CallSettings& c, LaunchPlan* 
     const int kw = a.kgroups == 1 ? 1 : ((a.kgroups + 3) / 4 * 4 <= (a.kgroups + 1) / 2 * 2 ? 4 : 2);
     opencnn::ConvArgs b = a;
     bool packed = false;
-    if (int e = pack_columns(&b, 4 / kw, (b.kgroups + kw - 1) / kw, (b.C + 7) / 8, kCutRanges, &packed)) return e;
-    REQUIRE(tile_with(b, kw));
+    const int chunks = (b.C + 7) / 8;
+    if (kw > 1 && split_into_pieces(chunks)) {
+      // workgroup tiles of 64 filters x 2 column tiles; kw = 4: the filter blocks come in pairs
+      const int kblocks = (b.kgroups + kw - 1) / kw * (kw / 2);
+      if (int e = pack_columns(&b, 2, kblocks, chunks, kCutRanges, &packed)) return e;
+      const long long colblocks = ((long long)b.colgroups + 1) / 2, nblocks = colblocks * kblocks;
+      REQUIRE(nblocks <= kMaxElems / 8);
+      b.nblocks = (int)nblocks;
+      b.colblocks = (int)colblocks;
+    } else {
+      if (int e = pack_columns(&b, 4 / kw, (b.kgroups + kw - 1) / kw, chunks, kCutRanges, &packed)) return e;
+      REQUIRE(tile_with(b, kw));
+    }
     int grid = 0;
-    if (int e = asm_grid(b, kw, (b.C + 7) / 8, kCutRanges, &grid)) return e;
+    if (int e = asm_grid(b, kw, chunks, kCutRanges, &grid)) return e;
     if (grid > 0)
       return launch_asm(b, kw, grid, ragged || b.kgroups % kw != 0, packed, lds_bytes(kw), st, plan);
     REQUIRE(variant != OPENCNN_KERNEL_ASM);

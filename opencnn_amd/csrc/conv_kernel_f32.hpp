@@ -369,14 +369,14 @@ __global__ void __launch_bounds__(256) wino_f32_fused(ConvArgs a) {
 // its partial result and raises a flag, the second adds its own on top.  a+b == b+a in fp32,
 // so the result does not depend on the arrival order.  The second wave only ever waits for a
 // wave that is already running its epilogue, never for one that has yet to be scheduled.
-constexpr int kMaxBalancedBlocks = 1024;
+constexpr int kMaxBalancedBlocks = 512;
 // [set][boundary between workgroups b and b+1][wave] -> {ticket, flag}; zero between launches
 // (the second contributor clears its pair).  Launches that may overlap in time must not share a
 // set: the host hands one to every stream that launches and to every stream capture (api.hip).
 constexpr int kEagerSets = 32;  // streams that launch directly
 constexpr int kGraphSets = 16;  // launches recorded into HIP graphs
 constexpr int kSyncSets = kEagerSets + kGraphSets;
-constexpr int kSyncWords = kMaxBalancedBlocks * 4 * 2;
+constexpr int kSyncWords = kMaxBalancedBlocks * 8 * 2;
 // (one more set at the end for launches that cut no tile: they are given it and never touch it)
 static __device__ unsigned g_split_sync[(kSyncSets + 1) * kSyncWords];
 

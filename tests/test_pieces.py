@@ -1,0 +1,200 @@
+"""The fp32 assembly kernels on bf16 pieces (opencnn_amd/csrc/gen_wino_f32_split_asm.py): CPU checks of the
+generator, and on the GPU the operands that bf16 pieces cannot hold."""
+import importlib.util
+import os
+import re
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "opencnn_amd", "csrc")
+CLANG = "/opt/rocm/lib/llvm/bin/clang"
+VARIANTS = [(False, False), (True, False), (True, True)]  # (ragged, packed)
+
+
+@pytest.fixture(scope="module")
+def split():
+    def load(name):
+        spec = importlib.util.spec_from_file_location(name, os.path.join(CSRC, name + ".py"))
+        mod = importlib.util.module_from_spec(spec)
+        sys.modules.setdefault(name, mod)
+        spec.loader.exec_module(mod)
+        return mod
+    load("gen_wino_f32_asm")
+    return load("gen_wino_f32_split_asm")
+
+
+@pytest.mark.parametrize("ragged,packed", VARIANTS)
+@pytest.mark.parametrize("kw", [2, 4])
+def test_kernel_text(split, kw, ragged, packed):
+    k = split.KernelSplit(kw, ragged, packed)
+    k.body()
+    text = "\n".join(k.lines)
+    assert k.vgpr_count <= 128 and k.sgpr_count <= 100  # two waves per SIMD: 128 + 128 accumulators
+    # four chunks (first / last of a segment or not) on pieces, two exact ones
+    assert text.count("v_mfma_f32_32x32x16_bf16") == 4 * 24
+    assert text.count("v_mfma_f32_32x32x2_f32") == 2 * 32
+    # the counted waits rely on STORES stores per output transform: plain, published, exact (and the NaNs
+    # of a part that pieces cannot hold)
+    assert text.count("buffer_store_dword") == 4 * split.STORES
+    assert all(int(n) <= 63 for n in re.findall(r"vmcnt\((\d+)\)", text))
+    assert all(int(n) <= 15 for n in re.findall(r"lgkmcnt\((\d+)\)", text))
+    labels = re.findall(r"^(\.L\w+):", text, re.M)
+    assert len(labels) == len(set(labels))
+    for target in re.findall(r"s_c?branch\w* (\.L\w+)", text):
+        assert target in labels
+    # MFMA operands start on even registers; an operand is split two instructions before it is read
+    lines = [l.strip() for l in k.lines]
+    for i, line in enumerate(lines):
+        if not line.startswith("v_mfma_f32_32x32x16"):
+            continue
+        reads = [(int(a), int(b)) for a, b in re.findall(r"v\[(\d+):(\d+)\]", line)]
+        assert all(a % 2 == 0 for a, _ in reads)
+        for back in lines[i - 2:i]:
+            m = re.match(r"v_(?!mfma)\w+ v(\d+),", back)
+            assert not m or back.startswith("s_nop") or lines[i - 1] == "s_nop 1" or \
+                not any(a <= int(m.group(1)) <= b for a, b in reads), (back, line)
+    # every wait for a flag is bounded, and the wave that gives up stores a 1 to the status word
+    polls = re.findall(r"^(\.L\w+_poll_\d+):", text, re.M)
+    assert len(polls) == 1
+    loop = lines[lines.index(polls[0] + ":"):][:14]
+    exits = [l.split()[-1] for l in loop if "s_cbranch" in l]
+    assert len(exits) == 2 and "_got_" in exits[0] and "_giveup_" in exits[1]
+    block = lines[lines.index(exits[1] + ":") + 1:][:5]
+    one = f"v{k.V['One']}"
+    assert block[0] == f"v_mov_b32 {one}, 1" and block[1] == "s_mov_b64 exec, 1"
+    assert block[2].split()[2].rstrip(",") == one and f"s[{k.S['Status']}:{k.S['Status'] + 1}]" in block[2]
+    assert block[4] == f"s_branch {exits[0]}"
+
+
+@pytest.mark.skipif(not os.path.exists(CLANG), reason="ROCm LLVM assembler not installed")
+def test_output_assembles_for_gfx950(tmp_path):
+    src = tmp_path / "k.s"
+    with open(src, "w") as f:
+        subprocess.run(["python3", os.path.join(CSRC, "gen_wino_f32_split_asm.py")], check=True, stdout=f)
+    subprocess.run([CLANG, "-x", "assembler", "-target", "amdgcn-amd-amdhsa", "-mcpu=gfx950", "-c", str(src),
+                    "-o", str(tmp_path / "k.o")], check=True)
+
+
+def test_waits_of_a_chunk_cover_its_loads(split):
+    """The counted waits, replayed: at every wait for a load of a steady-state chunk, the loads that may still be
+    in flight (the youngest vmcnt of them) do not include the ones the next split or transform reads."""
+    k = split.KernelSplit(2)
+    k.chunk(False, False)
+    lines = [l.strip() for l in k.lines]
+    one = [l for l in lines if l]
+    stream = one + one  # the second copy is the chunk in its steady state
+    inflight = []
+    for i, line in enumerate(stream):
+        m = re.match(r"buffer_load_dword(x4)? v\[?(\d+)", line)
+        if m:
+            first = int(m.group(2))
+            inflight.append(set(range(first, first + (4 if m.group(1) else 1))))
+        m = re.match(r"s_waitcnt vmcnt\((\d+)\)", line)
+        if m:
+            inflight = inflight[len(inflight) - min(int(m.group(1)), len(inflight)):]
+        if i >= len(one) and line.startswith("v_") and not line.startswith("v_mfma"):
+            regs = {int(r) for r in re.findall(r"\bv(\d+)\b", line)}
+            busy = set().union(*inflight) if inflight else set()
+            assert not regs & busy, (line, sorted(regs & busy))
+
+
+# ---------------------------------------------------------------- GPU
+# (N, C, H, W, K): three units with a ragged last one, an odd number of column groups, packed columns, tiles cut
+# between two workgroups, tiles cut among several, two filter blocks with a pair that is not full
+SHAPES = [(32, 17, 6, 6, 64), (32, 24, 5, 5, 100), (5, 33, 9, 9, 40), (64, 64, 40, 40, 64), (32, 256, 7, 7, 128),
+          (33, 40, 12, 13, 300)]
+
+
+def _run(ocn, torch, x, w):
+    C, H, W, N = x.shape
+    K = w.shape[3]
+    dev = torch.device("cuda:0")
+    guard = 1024
+    raw = torch.full((K * H * W * N + 2 * guard,), float("nan"), device=dev)
+    ws = torch.empty(ocn.workspace_bytes(C, K) // 4, device=dev)
+    ocn.conv_forward_desc(torch.from_numpy(x).to(dev), torch.from_numpy(w).to(dev), raw[guard:-guard], ws, N, C, H, W, K)
+    torch.cuda.synchronize()
+    assert "_asm_" in ocn.last_kernel()
+    assert torch.isnan(raw[:guard]).all() and torch.isnan(raw[-guard:]).all(), "wrote outside the output"
+    return raw[guard:-guard].cpu().numpy().reshape(K, H, W, N)
+
+
+def _tensors(shape, seed):
+    N, C, H, W, K = shape
+    rng = np.random.default_rng(seed)
+    return (rng.normal(size=(C, H, W, N)).astype(np.float32),
+            (rng.normal(size=(C, 3, 3, K)) * np.sqrt(2.0 / (9 * C))).astype(np.float32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES)
+def test_every_scale_of_the_operands(ocn, oracle, torch_gpu, shape):
+    # pieces hold 2^-108 ... 2^127; outside (and where outputs come out tiny or huge) the tiles are computed on the
+    # fp32 MFMA.  Relative to the fp64 direct convolution every scale has fp32's accuracy: C roundings of
+    # 2^-24 and the transforms' (below 1e-6 at these sizes); 2^-132 leaves 2^-17 of a denormal's bits.
+    x, w = _tensors(shape, 5)
+    want = oracle.direct_conv_f64(x, w).astype(np.float64)
+    for ex, ew in ((0, 0), (100, 0), (-100, 0), (0, -60), (-60, 40), (60, 60), (-115, 0), (0, -115), (-60, -60)):
+        print(f"scale {shape} 2^{ex} 2^{ew}", flush=True)
+        y = _run(ocn, torch_gpu, np.ldexp(x, ex), np.ldexp(w, ew)).astype(np.float64)
+        y = np.ldexp(y, -(ex + ew))
+        rel = np.linalg.norm(y - want) / np.linalg.norm(want)
+        assert rel <= 2e-6, (ex, ew, rel)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES)
+def test_operands_below_the_pieces(ocn, oracle, torch_gpu, shape):
+    # Denormal inputs that no bf16 piece holds (the sums on pieces are zero), in all channels, in the first or
+    # second half of them only (the other half zero: with a tile cut between workgroups, one part says
+    # nothing) or in one image; denormal filters; and zeros, which are exact as they are.
+    x, w = _tensors(shape, 6)
+    N, C, H, W, K = shape
+    tiny = np.float32(1e-41)
+    cases = {"inputs": (x * tiny, w), "filters": (x, w * tiny)}
+    for name, part in (("first half", slice(0, C // 2)), ("second half", slice(C // 2, C))):
+        z = np.zeros_like(x)
+        z[part] = x[part] * tiny
+        cases[name] = (z, w)
+    z = x.copy()
+    z[..., N // 2] *= tiny
+    cases["one image"] = (z, w)
+    for name, (xx, ww) in cases.items():
+        print(f"below the pieces {shape} {name}", flush=True)
+        y, direct = _run(ocn, torch_gpu, xx, ww), oracle.direct_conv_f64(xx, ww)
+        if name == "one image":  # the others have fp32's errors at their own scale
+            y, direct = y[..., N // 2], direct[..., N // 2]
+        # multiples of 2^-149: every halving of a transform and every sum rounds to that grid, fewer than 16 * C
+        # of them an output.  (An output within those steps of zero may come out as zero, hence no count of
+        # them; lost operands would leave no output at all.)
+        assert np.abs(y.astype(np.float64) - direct).max() <= 16 * C * 2.0 ** -149
+        assert (y != 0).mean() > 0.5
+    zero = w.copy()
+    zero[..., : K // 2] = 0
+    y = _run(ocn, torch_gpu, x, zero)
+    assert not y[: K // 2].any() and np.isfinite(y).all()
+    assert not _run(ocn, torch_gpu, np.zeros_like(x), w).any()
+    assert not _run(ocn, torch_gpu, x, np.zeros_like(w)).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES)
+def test_non_finite_operands_stay_in_their_tiles(ocn, oracle, torch_gpu, shape):
+    # An infinity in the last channel: the same non-finite elements as on the fp32 MFMA everywhere (the
+    # restatement of the reference's arithmetic), finite ones as accurate as ever.
+    N, C, H, W, K = shape
+    if H != W:
+        pytest.skip("the restatement takes square images")
+    x, w = _tensors(shape, 7)
+    x[C - 1, H // 2, 1, N - 1] = np.inf
+    x[0, 0, 0, 0] = np.nan
+    print(f"non-finite {shape}", flush=True)
+    y, want = _run(ocn, torch_gpu, x, w), oracle.winograd_f32(x, w)
+    assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(np.isposinf(y), np.isposinf(want))
+    ok = np.isfinite(want)
+    rel, _, _ = oracle.compare(np.where(ok, y, 0.0), np.where(ok, want, 0.0))
+    assert rel <= 2e-6, rel
