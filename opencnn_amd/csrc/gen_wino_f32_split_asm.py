@@ -393,12 +393,17 @@ class KernelSplit(Kernel):
         self.e(f"s_xor_b32 {self.sr('Buf')}, {self.sr('Buf')}, 0x{BUFFER_SWAP:x}")
 
     # ------------------------------------------------------------------ one chunk
+    # (filter group, column group) of the MFMAs, three each, for the wave's first and second position.  The
+    # orders leave A0 and B0 early in the first half, A1 early in the second, so that the filter
+    # registers are free, and loaded again, half a unit before their next split.
+    ORDER = [[(0, 0), (0, 1), (1, 0), (1, 1)], [(0, 0), (1, 0), (0, 1), (1, 1)]]
     # What rides behind MFMA i, as (first slot, last slot + 1) per piece of work.  A split ends in front of
     # the first MFMA that reads it (3, 6, 12, 12, 15, 18; A0 and B0 of the next unit: the next chunk) and
     # starts behind the last one that reads the registers it overwrites.
-    SLOTS = {"cursors": (0, 2), "column": (2, 6), "patch": (3, 19), "row": (6, 12),
-             "B1": (0, 3), "A1": (3, 6), "A0'": (6, 9), "U0": (9, 10), "B0'": (9, 12), "B1'": (12, 15),
-             "swap": (15, 16), "read": (16, 18), "exchange": (17, 24), "A1'": (15, 18), "U1": (18, 19), "A0": (18, 21), "B0": (21, 24)}
+    SLOTS = {"cursors": (0, 2), "column": (2, 6), "patch": (3, 11), "row": (6, 12),
+             "B1": (0, 3), "A1": (3, 6), "A0'": (6, 9), "U0": (9, 10), "B0'": (9, 12), "A1'": (12, 15), "U1": (15, 16),
+             "B1'": (15, 18), "swap": (14, 15), "read": (15, 16), "read'": (18, 19), "B0": (18, 21), "A0": (21, 24),
+             "exchange": (17, 24)}
 
     def captured(self, *emitters):
         main, self.lines = self.lines, []
@@ -461,7 +466,7 @@ class KernelSplit(Kernel):
         put("cursors", self.captured(self.advance_p, self.channel_descriptor, self.advance_q, self.filter_offsets))
         put("B1", b1(0))
         put("column", [("wait", "P")] + column)
-        put("patch", [("vm", "P", self.patch_load("P", p)) for p in range(16)])
+        put("patch", [("vm", "P", self.patch_load("P", 4 * r + c)) for c in range(4) for r in range(4)])
         put("A1", [("wait", "U1")] + split(self.u_raw(0, 1), "A", self.V["A1"]))
         put("A0'", a0(1))
         put("U0", self.u_load_items(0))
@@ -472,7 +477,8 @@ class KernelSplit(Kernel):
         put("A1'", split(self.u_raw(1, 1), "A", self.V["A1"]))
         put("U1", self.u_load_items(1))
         if not last:
-            put("read", self.read_items())
+            put("read", self.read_items()[:4])
+            put("read'", self.read_items()[4:])
             put("A0", a0(0))
             put("B0", b0(0))
         else:
@@ -483,14 +489,13 @@ class KernelSplit(Kernel):
             seq = self.read_items() + a0(0) + b0(0)
         i = 0
         for e in range(2):
-            for kg in range(2):
-                for cg in range(2):
-                    for prod in range(3):
-                        if i in (0, 3, 6, 12, 15, 18):
-                            seq.append("s_nop 1")  # two wait states between a split and the MFMA that reads it
-                        seq.append(self.mfma(e, kg, cg, prod, first))
-                        seq += fill[i]
-                        i += 1
+            for kg, cg in self.ORDER[e]:
+                for prod in range(3):
+                    if i in (0, 3, 6, 12, 15, 18):
+                        seq.append("s_nop 1")  # two wait states between a split and the MFMA that reads it
+                    seq.append(self.mfma(e, kg, cg, prod, first))
+                    seq += fill[i]
+                    i += 1
         self.emit_chunk(seq, first)
         self.e(f"s_add_u32 {self.sr('G')}, {self.sr('G')}, 1")
         self.e(f"s_add_u32 {self.sr('Cm')}, {self.sr('Cm')}, 1")
