@@ -645,38 +645,24 @@ class KernelSplit(Kernel):
                     for q in range(4):
                         e(f"buffer_store_dword {out(q, b)}, {self.vr('Eff', q)}, {self.sr('RsrcY', 4)}, 0 offen nt")
                 continue
-            plain, stored, nomerge = self.newlabel("store"), self.newlabel("stored"), self.newlabel("nomerge")
+            plain, stored, merges = self.newlabel("store"), self.newlabel("stored"), self.newlabel("merges")
             e(f"s_bitcmp1_b32 {self.sr('Kind')}, 1")
-            e(f"s_cbranch_scc0 {nomerge}")
-            if kg == 0:
-                self.wait_flag()
-            for b in range(4):
-                self.row_descriptor(kg, b)
-                for q in range(4):
-                    e(f"buffer_load_dword {m(8 + q, b)}, {self.vr('Eff', q)}, {self.sr('RsrcY', 4)}, 0 offen sc0 sc1")
-            e("s_waitcnt vmcnt(0)")
-            if kg == 1:
-                self.store_flag(self.vr("Zero"))  # hand the flag back for the next launch
-            for b in range(4):
-                for q in range(4):
-                    e(f"v_add_f32 {out(q, b)}, {out(q, b)}, {m(8 + q, b)}")
-            self.label(nomerge)
+            e(f"s_cbranch_scc1 {merges}")
             for b in range(4):
                 for q in range(4):
                     e(f"v_add_f32 {self.vr('Sum')}, {self.vr('Sum')}, |{out(q, b)}|")
-            e(f"s_bitcmp1_b32 {self.sr('Kind')}, 0")
-            e(f"s_cbranch_scc0 {plain}")
-            for b in range(4):
-                self.row_descriptor(kg, b)
-                for q in range(4):
-                    e(f"buffer_store_dword {out(q, b)}, {self.vr('Eff', q)}, {self.sr('RsrcY', 4)}, 0 offen sc0 sc1")
-            e(f"s_branch {stored}")
-            self.label(plain)
-            for b in range(4):
-                self.row_descriptor(kg, b)
-                for q in range(4):
-                    e(f"buffer_store_dword {out(q, b)}, {self.vr('Eff', q)}, {self.sr('RsrcY', 4)}, 0 offen nt")
-            self.label(stored)
+            self.store_rows(kg, out, plain, stored)
+            main, self.lines = self.lines, []
+            self.label(merges)
+            if kg == 0:
+                for b in range(4):
+                    for q in range(4):
+                        e(f"v_mov_b32 {self.vr('VOFF', 4 * b + q)}, {out(q, b)}")
+                e(f"s_branch {stored}")
+            else:
+                self.merge(out, stored)
+            self.outofline.extend(self.lines)
+            self.lines = main
         if exact:
             return
         # M = lanes whose sum says that the pieces may not have held the operands: not finite (or close
@@ -726,6 +712,49 @@ class KernelSplit(Kernel):
         self.filters_are_zero(zero, zero_done)
         self.outofline.extend(self.lines)
         self.lines = main
+
+    def store_rows(self, kg, out, plain, stored):
+        """The 16 outputs of filter group kg: published past the caches (Kind bit 0), or final ones."""
+        for policy in (" sc0 sc1", " nt"):
+            if policy == " nt":
+                self.label(plain)
+            else:
+                self.e(f"s_bitcmp1_b32 {self.sr('Kind')}, 0")
+                self.e(f"s_cbranch_scc0 {plain}")
+            for b in range(4):
+                self.row_descriptor(kg, b)
+                for q in range(4):
+                    self.e(f"buffer_store_dword {out(q, b)}, {self.vr('Eff', q)}, {self.sr('RsrcY', 4)}, 0 offen{policy}")
+            if policy != " nt":
+                self.e(f"s_branch {stored}")
+        self.label(stored)
+
+    def merge(self, out1, done):
+        """A range that ends inside a tile: its last segment.  Both filter groups' outputs are there (those of
+        group 0 in VOFF, which nothing reads any more) before the wait for the flag, so that between the flag
+        of the workgroup behind and this one's there is one trip to memory and its acknowledgement: the
+        partial tile lands in P and U, once their last prefetches have.  (With the two groups merged one after
+        the other, a trip each, a hand-over took 1.7 us longer.)"""
+        e = self.e
+        out0 = lambda q, b: self.vr("VOFF", 4 * b + q)
+        land = lambda kg, q, b: self.vr("P" if kg == 0 else "U", 4 * b + q)
+        e("s_waitcnt vmcnt(0)")
+        self.wait_flag()
+        for kg in range(2):
+            for b in range(4):
+                self.row_descriptor(kg, b)
+                for q in range(4):
+                    e(f"buffer_load_dword {land(kg, q, b)}, {self.vr('Eff', q)}, {self.sr('RsrcY', 4)}, 0 offen sc0 sc1")
+        for kg, out in ((0, out0), (1, out1)):
+            e("s_waitcnt vmcnt(16)")  # the group's loads (behind them: the other group's, or 16 stores)
+            for b in range(4):
+                for q in range(4):
+                    e(f"v_add_f32 {out(q, b)}, {out(q, b)}, {land(kg, q, b)}")
+                    e(f"v_add_f32 {self.vr('Sum')}, {self.vr('Sum')}, |{out(q, b)}|")
+            if kg == 1:
+                self.store_flag(self.vr("Zero"))  # hand the flag back for the next launch
+            self.store_rows(kg, out, self.newlabel("store"), self.newlabel("stored"))
+        e(f"s_branch {done}")
 
     def filters_are_zero(self, entry, done):
         """Sums of zero with inputs that are not: fine when the wave's eight filters are zero (or do not

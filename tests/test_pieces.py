@@ -37,9 +37,10 @@ def test_kernel_text(split, kw, ragged, packed):
     # four chunks (first / last of a segment or not) on pieces, two exact ones
     assert text.count("v_mfma_f32_32x32x16_bf16") == 4 * 24
     assert text.count("v_mfma_f32_32x32x2_f32") == 2 * 32
-    # the counted waits rely on STORES stores per output transform: plain, published, exact (and the NaNs
-    # of a part that pieces cannot hold)
-    assert text.count("buffer_store_dword") == 4 * split.STORES
+    # the counted waits rely on STORES stores per output transform: plain, published, merged, merged and
+    # published, exact (and the NaNs of a part that pieces cannot hold)
+    assert text.count("buffer_store_dword") == 6 * split.STORES
+    assert len(re.findall(r"buffer_load_dword v\d+, [^\n]* sc0 sc1", text)) == 32  # a partial tile
     assert all(int(n) <= 63 for n in re.findall(r"vmcnt\((\d+)\)", text))
     assert all(int(n) <= 15 for n in re.findall(r"lgkmcnt\((\d+)\)", text))
     labels = re.findall(r"^(\.L\w+):", text, re.M)
