@@ -735,15 +735,24 @@ int pack_columns(opencnn::ConvArgs* a, int cw, int kblocks, int chunks, CutTiles
 }
 
 // fp32 assembly kernels, balanced split: which weight of a tile's output transform (half units,
-// 0 = equal numbers of units) lets the slowest range end first.  A range costs its units, 1.3
-// units per tile it touches (output transform, restart of the pipeline), 1.0 when it starts inside
-// a tile (that part is published through memory) and 0.6 when it ends inside one (it waits for the
-// published part): fitted to the kernels' times on twelve layers under every weight; the choice
-// it makes there is never slower than the equal split and up to 6.7 % faster (tiles of 8 units,
-// 1.5 - 2.3 tiles per range).  Cached per thread: a network has a handful of distinct lines.
-int choose_range_weight(int tiles, int chunks, int ranges) {
+// 0 = equal numbers of units) lets the slowest range end first.  A range costs its units, and in tenths of a
+// unit: so much per tile it touches (output transform, restart of the pipeline), when it starts inside a tile
+// (that part is published through memory) and when it ends inside one (it waits for the published part).
+// On the fp32 MFMA: fitted to the kernels' times on twelve layers under every weight; the choice it makes
+// there is never slower than the equal split and up to 6.7 % faster (tiles of 8 units, 1.5 - 2.3 tiles per
+// range).  On pieces the units are shorter and the output transform longer: fitted to ten layers under the
+// weights 0 ... 6, within 1 % of the best weight on all of them but one (with the other kernel's costs up to
+// 5.4 % off: N=96 C=K=256 14x14 75.2 us at weight 0, 70.7 at 5; N=32 C=K=64 56x56 32.1 at 2, 30.8 at 6).
+// Cached per thread: a network has a handful of distinct lines.
+struct RangeCosts {
+  int tile, starts_inside, ends_inside, max_weight;
+};
+constexpr RangeCosts kRangeCosts[2] = {{13, 10, 6, 4}, {22, 4, 6, 6}};  // fp32 MFMA, pieces
+
+int choose_range_weight(int tiles, int chunks, int ranges, bool pieces) {
+  const RangeCosts& costs = kRangeCosts[pieces];
   struct Entry {
-    int tiles, chunks, ranges, weight;
+    int tiles, chunks, ranges, weight;  // (the chunks say which kernel)
   };
   thread_local Entry cache[16] = {};
   thread_local unsigned next = 0;
@@ -752,7 +761,7 @@ int choose_range_weight(int tiles, int chunks, int ranges) {
   // (a weight has to promise half a percent to replace the equal split, and more than a smaller weight)
   long long best_cost = 0;
   int best = 0;
-  for (int weight = 0; weight <= 4; ++weight) {
+  for (int weight = 0; weight <= costs.max_weight; ++weight) {
     // weight 0: the kernel deals whole units; else half units on the weighted line (weighted_unit_range
     // of the generator)
     const long long vt = weight ? 2LL * chunks + weight : chunks, total = (long long)tiles * vt;
@@ -768,9 +777,9 @@ int choose_range_weight(int tiles, int chunks, int ranges) {
     for (int r = 0; r < ranges; ++r) {
       const long long end = unit_at(r + 1);
       if (end > begin) {
-        long long cost = 10 * (end - begin) + 13 * ((end - 1) / chunks - begin / chunks + 1);  // tenths of a unit
-        if (begin % chunks) cost += 10;
-        if (end % chunks) cost += 6;
+        long long cost = 10 * (end - begin) + costs.tile * ((end - 1) / chunks - begin / chunks + 1);  // tenths of a unit
+        if (begin % chunks) cost += costs.starts_inside;
+        if (end % chunks) cost += costs.ends_inside;
         if (cost > slowest) slowest = cost;
       }
       begin = end;
@@ -814,7 +823,7 @@ int launch_asm(const opencnn::ConvArgs& a, int kw, int grid, bool ragged, bool p
   l.c_real_or_mode = a.C;
   // Ranges of the balanced split that are at least a tile long may be cut on a weighted line.
   if (grid < a.nblocks && a.sync != nullptr)
-    l.range_weight = t_range_weight >= 0 ? t_range_weight : choose_range_weight(a.nblocks, l.chunks, grid);
+    l.range_weight = t_range_weight >= 0 ? t_range_weight : choose_range_weight(a.nblocks, l.chunks, grid, pieces);
   return launch_asm_kernel(a, l, st, plan);
 }
 
