@@ -1163,9 +1163,19 @@ int launch_on_flag_set(opencnn::ConvArgs& a, const CallSettings& c, LaunchPlan* 
     // The assembly kernels take a last filter block with fewer than kw filter groups: a wave
     // without filters reads zeros past the end of Ww, multiplies them and stores no row (the
     // row masks of the _ragged kernels).  So: the kw that leaves the fewest such waves, 4 on a tie.
-    // A single filter group would idle half of the matrix pipes: the register variant below
-    // is faster there (measured, K = 32).
-    const int kw = a.kgroups == 1 ? 1 : ((a.kgroups + 3) / 4 * 4 <= (a.kgroups + 1) / 2 * 2 ? 4 : 2);
+    // A single filter group idles half of the tile: the register variant below is faster (measured, K = 32)
+    // unless its workgroups of 128 columns leave half of the compute units without work, which it cannot
+    // cut.  Fused kernel in us, register variant / pieces: its workgroups 196: N=32 C=64 56x56 26.7 / 29.7,
+    // N=128 C=128 28x28 48.4 / 49.4; 98: N=64 C=20 28x28 13.0 / 10.1; 49: N=128 C=64 14x14 22.5 / 15.8; 21:
+    // N=16 C=512 18x18 162 / 31.5.
+    int kw = (a.kgroups + 3) / 4 * 4 <= (a.kgroups + 1) / 2 * 2 ? 4 : 2;
+    if (a.kgroups == 1) {
+      int cus = 0;
+      if (int e = compute_units(&cus)) return e;
+      const long long columns = (long long)a.tiles_h * a.tiles_w * a.N;
+      const bool few = (columns + 127) / 128 <= cus / 2;
+      kw = variant == OPENCNN_KERNEL_AUTO && split_into_pieces((a.C + 7) / 8) && few ? 2 : 1;
+    }
     opencnn::ConvArgs b = a;
     bool packed = false;
     const int chunks = (b.C + 7) / 8;

@@ -105,9 +105,10 @@ def test_waits_of_a_chunk_cover_its_loads(split):
 
 # ---------------------------------------------------------------- GPU
 # (N, C, H, W, K): three units with a ragged last one, an odd number of column groups, packed columns, tiles cut
-# between two workgroups, tiles cut among several, two filter blocks with a pair that is not full
+# between two workgroups, tiles cut among several, two filter blocks with a pair that is not full, a single group
+# of filters
 SHAPES = [(32, 17, 6, 6, 64), (32, 24, 5, 5, 100), (5, 33, 9, 9, 40), (64, 64, 40, 40, 64), (32, 256, 7, 7, 128),
-          (33, 40, 12, 13, 300)]
+          (33, 40, 12, 13, 300), (16, 136, 9, 9, 32), (3, 20, 14, 11, 7)]
 
 
 def _run(ocn, torch, x, w):
