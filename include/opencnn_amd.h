@@ -361,7 +361,8 @@ const char *opencnn_last_error(void);
 /*
  * Name of the fused kernel that this thread's last successful launch used ("" before the first):
  * a short static string such as "wino_f32_asm_kw2" or "wino_f16_asm_kw4_packed" (the assembly
- * kernels' symbol names) or "wino_f32_fused_lds" (a HIP C++ kernel).  For logs and tests: which
+ * kernels' symbol names; the fp32 ones exist twice under the same names, multiplying bf16 pieces from
+ * 17 channels on) or "wino_f32_fused_lds" (a HIP C++ kernel).  For logs and tests: which
  * kernel family a shape ends up in is the library's choice (see opencnn_set_kernel_variant).
  * No counterpart in the reference, whose single kernel is fixed at compile time.
  */

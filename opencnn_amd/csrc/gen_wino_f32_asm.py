@@ -2,7 +2,9 @@
 """Generator of the hand-scheduled gfx950 assembly of the fused Winograd F(2x2,3x3) kernel.
 
 Emits one kernel per KW (waves of a workgroup that share a column tile), wino_f32_asm_kw2 and
-wino_f32_asm_kw4, each also as a _ragged variant for shapes outside the reference's tiling.
+wino_f32_asm_kw4, each also as a _ragged variant for shapes outside the reference's tiling.  Layers of
+up to 16 channels run them; deeper ones the kernels of gen_wino_f32_split_asm.py, which extend the
+class below.
 Same mathematics and data layout as wino_f32_stream in conv_kernel_f32.hpp (which replaces the
 reference's Winograd_kernel, src/convolutionForward_32x64x8.cu:169-262); what the assembly adds
 is control over the things hipcc does not let the C++ source decide:

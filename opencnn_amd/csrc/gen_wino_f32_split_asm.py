@@ -15,11 +15,18 @@ them.  Against 64 bits the sums are nearer than those of the fp32 MFMA (relative
 dot product over 64 / 512 / 1024 channels: 1.1e-7 / 3.4e-7 / 4.9e-7 against 1.5e-7 / 4.1e-7 /
 5.7e-7): there are fewer roundings on the way.
 
-What the pieces cannot hold: an infinity or NaN (its residual is NaN), and the low bits of values
-below 2^-108 (bf16 has no exponents below fp32's).  A workgroup therefore sums the magnitudes of the
-outputs it stores, per lane; when a sum is not finite, or is not zero and below 2^-64, the workgroup
-computes the tiles it has stored once more with v_mfma_f32_32x32x2_f32 (`exact`), which is what the
-rest of this family always does, and stores them again.
+What the pieces cannot hold: an infinity or NaN (its residual is NaN), the low bits of values below
+2^-108 and all of values below 2^-134 (bf16 has no exponents below fp32's).  A lane therefore sums the
+magnitudes of the outputs it stores; when a sum is not finite, or is not zero and below 2^-64, or is
+zero although the column's input (Nz) and the filters are not, the workgroup computes the tiles that
+it stores once more with v_mfma_f32_32x32x2_f32 (exact_chunk), which is what gen_wino_f32_asm.py's
+kernels always use, and stores them again.
+
+What bounds it: power on layers that fill the chip (N=128 C=K=512 7x7 runs at 2.03 GHz, the fp32 MFMA
+kernel at 2.49; with every wait taken out it takes as long, at a lower clock), issue on small ones (two
+waves per SIMD, some 360 instructions a unit each; without its MFMAs a unit takes 96 % of the time).
+Fused kernel on the fp32 MFMA / here, us: N=64 C=K=64 56x56 65 / 55, N=128 C=K=128 28x28 110 / 94,
+C=K=256 14x14 106 / 92, C=K=512 7x7 128 / 106, N=1 C=K=64 14x14 22.3 / 17.1.
 
 Workgroup: eight waves, one tile of 64 filters x 64 columns (2 x 2 MFMA tiles) for all 16 positions.
 Wave w holds positions 2w and 2w + 1: every U and every V element is read, and split, by one wave of
