@@ -15,12 +15,19 @@ them.  Against 64 bits the sums are nearer than those of the fp32 MFMA (relative
 dot product over 64 / 512 / 1024 channels: 1.1e-7 / 3.4e-7 / 4.9e-7 against 1.5e-7 / 4.1e-7 /
 5.7e-7): there are fewer roundings on the way.
 
-What the pieces cannot hold: an infinity or NaN (its residual is NaN), the low bits of values below
-2^-108 and all of values below 2^-134 (bf16 has no exponents below fp32's).  A lane therefore sums the
-magnitudes of the outputs it stores; when a sum is not finite, or is not zero and below 2^-64, or is
-zero although the column's input (Nz) and the filters are not, the workgroup computes the tiles that
-it stores once more with v_mfma_f32_32x32x2_f32 (exact_chunk), which is what gen_wino_f32_asm.py's
-kernels always use, and stores them again.
+Range: bf16 has no exponents below fp32's, so the pieces of a value below 2^-110 would fall off the end of
+bf16's grid, 2^-133.  Every operand is therefore split times 2^16: fp32's own grid, 2^-149, then lies on
+bf16's, and the pieces are exact for every value up to 2^112.  The outputs are stored times 2^-32.  V gets
+its factor in the input transform (six instructions a patch), U in front of its split (one a value):
+14 of 241 vector instructions a unit, 0.7 ... 2.4 % of a call (N=1 C=K=64 14x14 19.7 -> 20.2 us,
+N=128 C=K=512 7x7 106.6 -> 107.4).  Deciding by the magnitude of operands or outputs instead where the pieces would lose
+bits takes both operands' largest and smallest values, of all waves; an output's neighbours do not tell.
+
+What the pieces cannot hold: infinities and NaNs (their residual is NaN), operands of 2^112 or more and
+outputs of 2^94 or more (infinite once scaled).  A lane therefore sums the magnitudes of the outputs it stores;
+where a sum is not finite, or close to it, the workgroup computes the tiles that it stores once more with
+v_mfma_f32_32x32x2_f32 (exact_chunk), which is what gen_wino_f32_asm.py's kernels always use, and
+stores them again.
 
 What bounds it: power on layers that fill the chip (N=128 C=K=512 7x7 runs at 2.03 GHz, the fp32 MFMA
 kernel at 2.49; with every wait taken out it takes as long, at a lower clock), issue on small ones (two
@@ -51,7 +58,8 @@ BUFFER_SWAP = 0x20000       # the two V buffers: bytes 0 .. 32K and 128K .. 160K
 LDS_BYTES = 160 * 1024
 STORES = 32                 # stores of an output transform, per wave
 SUM_LARGE = 0x7E800000      # 2^126
-SUM_TINY = 0x1F800000       # 2^-64
+SCALE = 0x47800000          # 2^16, on U and on V
+UNSCALE = 0x2F800000        # 2^-32
 
 
 class KernelSplit(Kernel):
@@ -79,7 +87,7 @@ class KernelSplit(Kernel):
         self.S.update(X=8, U=10, Y=12, Sync=14, Status=4, SpinLimit=6)
         for n in ["L", "Wave", "Begin", "Nunits", "G", "Tp", "Cp", "Tq", "Cq", "Tm", "Cm",
                   "SegEnd", "Kind", "ColStep", "RowStep", "Uoff0", "Uoff1",
-                  "Dkb", "DkbPrev", "DkbM", "Spin", "Stamps", "Bad", "Buf", "MaskHi", "PlaceTn"]:
+                  "Dkb", "DkbPrev", "DkbM", "Spin", "Stamps", "Bad", "Buf", "MaskHi", "Scale", "PlaceTn"]:
             self.S[n] = S.get(n)
         self.S["RsrcX"] = S.get("RsrcX", 4, 4)
         self.S["RsrcU"] = S.get("RsrcU", 4, 4)
@@ -94,7 +102,7 @@ class KernelSplit(Kernel):
         V = Alloc(1, 128)
         self.V = {}
         for n, cnt, al in [("Lane16", 1, 1), ("Lds0", 1, 1), ("Lds1", 1, 1), ("LdsWr", 1, 1),
-                           ("Nz", 1, 1), ("NzNext", 1, 1), ("EffP", 1, 1), ("EffPrev", 1, 1), ("Tmp", 2, 1), ("Eff", 4, 1),
+                           ("EffP", 1, 1), ("EffPrev", 1, 1), ("Tmp", 2, 1), ("Eff", 4, 1),
                            ("Sum", 1, 1), ("VOFF", 16, 1), ("P", 16, 1), ("U", 16, 4),
                            # 64 registers that hold nothing between two chunks: the output transform's
                            ("EX", 64, 4)]:
@@ -334,11 +342,12 @@ class KernelSplit(Kernel):
     # ------------------------------------------------------------------ pieces of a chunk
     def split_operand(self, raw, kind, dst):
         """Instructions that turn four fp32 registers (channels of the lane half, in pairs) into bf16
-        pieces: A = [l l h h m m], B = [h h m m h h l l] (two registers per piece)."""
+        pieces: A = [l l h h m m], B = [h h m m h h l l] (two registers per piece).  A (filters) is scaled
+        here, B was in the transform."""
         x = lambda i: v(raw[i])
         t = lambda i: self.vr("S4", i)
         h, m, l = ((2, 4, 0) if kind == "A" else (0, 2, 6))
-        out = []
+        out = [f"v_mul_f32 {x(i)}, {self.sr('Scale')}, {x(i)}" for i in range(4)] if kind == "A" else []
         for q in range(2):
             out.append(f"v_cvt_pk_bf16_f32 {v(dst + h + q)}, {x(2 * q)}, {x(2 * q + 1)}")
         for piece, nxt in ((h, m), (m, l)):
@@ -371,24 +380,35 @@ class KernelSplit(Kernel):
         c = "0" if fresh and prod == 0 else self.acc(e, kg, cg, 0, 16)
         return f"v_mfma_f32_32x32x16_bf16 {self.acc(e, kg, cg, 0, 16)}, {v(ar, 4)}, {v(br, 4)}, {c}"
 
-    def transform_items(self, src, fresh):
+    def transform_items(self, src, exact):
         """V = B^T d B of the patch in src (columns first, as Kernel.transform; the rows in place, v0 the
-        one register more), and its way into the write buffer: two positions an instruction.  The bits of
-        the patch are collected in Nz, or (fresh: the first unit of the next segment) in NzNext."""
+        one register more), and its way into the write buffer: two positions an instruction.  Unless exact,
+        V comes out scaled, with the roundings of a transform that is not (a power of two): of every pair of terms
+        one is scaled and the other meets the factor in an fma.  Rows 0 .. 2 are scaled in the column pass (one
+        term serves all three), row 3 in the row pass (two terms serve its four): six multiplications a patch."""
         d = lambda i: self.vr(src, i)
-        nz = self.vr("NzNext" if fresh else "Nz")
         t = lambda i: self.vr("T", i)
+        scale = self.sr("Scale")
+        scaled = lambda x: f"v_mul_f32 {x}, {scale}, {x}"
         column, row = [], []
         for c in range(4):
-            column += [f"v_sub_f32 {t(c)}, {d(c)}, {d(8 + c)}", f"v_add_f32 {t(4 + c)}, {d(4 + c)}, {d(8 + c)}",
-                       f"v_sub_f32 {t(8 + c)}, {d(8 + c)}, {d(4 + c)}", f"v_sub_f32 {t(12 + c)}, {d(4 + c)}, {d(12 + c)}",
-                       f"v_or3_b32 {nz}, {d(c)}, {d(4 + c)}, {'0' if fresh and c == 0 else nz}",
-                       f"v_or3_b32 {nz}, {d(8 + c)}, {d(12 + c)}, {nz}"]
+            if exact:
+                column += [f"v_sub_f32 {t(c)}, {d(c)}, {d(8 + c)}", f"v_add_f32 {t(4 + c)}, {d(4 + c)}, {d(8 + c)}",
+                           f"v_sub_f32 {t(8 + c)}, {d(8 + c)}, {d(4 + c)}"]
+            else:
+                column += [scaled(d(8 + c)), f"v_fma_f32 {t(c)}, {d(c)}, {scale}, -{d(8 + c)}",
+                           f"v_fma_f32 {t(4 + c)}, {d(4 + c)}, {scale}, {d(8 + c)}",
+                           f"v_fma_f32 {t(8 + c)}, -{d(4 + c)}, {scale}, {d(8 + c)}"]
+            column.append(f"v_sub_f32 {t(12 + c)}, {d(4 + c)}, {d(12 + c)}")
         for r in range(4):
             m = [t(4 * r + c) for c in range(4)]
             put = lambda p, x, y: ("lds", "write", f"ds_write2st64_b32 {self.vr('LdsWr')}, {x}, {y} offset0:{8 * p} offset1:{8 * p + 8}")
-            row += [f"v_add_f32 v0, {m[1]}, {m[2]}", f"v_sub_f32 {m[0]}, {m[0]}, {m[2]}",
-                    f"v_sub_f32 {m[3]}, {m[1]}, {m[3]}", put(4 * r, m[0], "v0"),
+            if exact or r < 3:
+                outer = [f"v_sub_f32 {m[0]}, {m[0]}, {m[2]}", f"v_sub_f32 {m[3]}, {m[1]}, {m[3]}"]
+            else:
+                row += [scaled(m[1]), scaled(m[2])]
+                outer = [f"v_fma_f32 {m[0]}, {m[0]}, {scale}, -{m[2]}", f"v_fma_f32 {m[3]}, -{m[3]}, {scale}, {m[1]}"]
+            row += [f"v_add_f32 v0, {m[1]}, {m[2]}", *outer, put(4 * r, m[0], "v0"),
                     f"v_sub_f32 {m[2]}, {m[2]}, {m[1]}", put(4 * r + 2, m[2], m[3])]
         return column, row
 
@@ -469,7 +489,7 @@ class KernelSplit(Kernel):
         a0 = lambda e: [("wait", "U0")] * (e == 0) + split(self.u_raw(e, 0), "A", self.V["A0"])
         b0 = lambda e: [("lwait", f"V{e}0")] + split(self.v_raw(e, 0), "B", self.V["B0"])
         b1 = lambda e: [("lwait", f"V{e}1")] + split(self.v_raw(e, 1), "B", self.V["B1"])
-        column, row = self.transform_items("P", last)
+        column, row = self.transform_items("P", False)
         put("cursors", self.captured(self.advance_p, self.channel_descriptor, self.advance_q, self.filter_offsets))
         put("B1", b1(0))
         put("column", [("wait", "P")] + column)
@@ -510,7 +530,7 @@ class KernelSplit(Kernel):
     def exact_chunk(self, first):
         """Unit G on the fp32 MFMA, one piece of work after the other."""
         self.comment(f"---- exact chunk{', first of a segment' if first else ''}")
-        column, row = self.transform_items("P", False)
+        column, row = self.transform_items("P", True)
         seq = self.read_items() + [("wait", "U1"), ("lwait", "V11")]
         seq += self.captured(self.advance_p, self.channel_descriptor, self.advance_q, self.filter_offsets)
         for e in range(2):
@@ -672,26 +692,12 @@ class KernelSplit(Kernel):
             self.lines = main
         if exact:
             return
-        # M = lanes whose sum says that the pieces may not have held the operands: not finite (or close
-        # to it), or not zero and tiny
-        mm, tt = self.sr("M", 2), s(self.S["T"] + 2, 2)
-        zero, zero_done, bad, bad_done, flag, done = (self.newlabel(x) for x in ("zero", "zerodone", "bad", "baddone", "flag", "nosplit"))
+        # a lane whose sum is not finite (or close to it): the workgroup computes the tiles that it stores again.
+        # A part that is published carries its infinities and NaNs to the workgroup that stores the tile.
+        bad, bad_done, flag, done = (self.newlabel(x) for x in ("bad", "baddone", "flag", "nosplit"))
         e(f"s_mov_b32 {t(0)}, 0x{SUM_LARGE:x}")
-        e(f"s_mov_b32 {t(1)}, 0x{SUM_TINY:x}")
-        e(f"v_cmp_ngt_f32 {mm}, {t(0)}, {self.vr('Sum')}")
-        e(f"v_cmp_gt_f32 {tt}, {t(1)}, {self.vr('Sum')}")
-        e(f"v_cmp_lt_f32 vcc, 0, {self.vr('Sum')}")
-        e(f"s_and_b64 {tt}, {tt}, vcc")
-        e(f"s_or_b64 {mm}, {mm}, {tt}")
-        # a sum of zero although the column's input is not
-        e(f"v_lshlrev_b32 {self.vr('Tmp')}, 1, {self.vr('Nz')}")
-        e(f"v_cmp_ne_u32 {tt}, 0, {self.vr('Tmp')}")
-        e(f"v_cmp_eq_f32 vcc, 0, {self.vr('Sum')}")
-        e(f"s_and_b64 vcc, vcc, {tt}")
-        e(f"s_cbranch_scc1 {zero}")
-        self.label(zero_done)
-        e(f"s_cmp_lg_u64 {mm}, 0")
-        e(f"s_cbranch_scc1 {bad}")
+        e(f"v_cmp_ngt_f32 vcc, {t(0)}, {self.vr('Sum')}")
+        e(f"s_cbranch_vccnz {bad}")
         self.label(bad_done)
         e(f"s_bitcmp1_b32 {self.sr('Kind')}, 0")
         e(f"s_cbranch_scc1 {flag}")
@@ -702,26 +708,16 @@ class KernelSplit(Kernel):
         self.flag_address(True)
         self.store_flag(self.vr("One"))
         e(f"s_branch {done}")
-        # bad lanes: the workgroup computes its tiles again; a published part tells the workgroup that stores
-        # the tile, with NaNs
         self.label(bad)
-        e(f"s_mov_b32 {self.sr('Bad')}, 1")
         e(f"s_bitcmp1_b32 {self.sr('Kind')}, 0")
-        e(f"s_cbranch_scc0 {bad_done}")
-        e(f"s_mov_b32 {self.sr('Bad')}, 0")
-        e(f"v_mov_b32 {self.vr('Sum')}, 0x7fc00000")
-        for kg in range(2):
-            for b in range(4):
-                self.row_descriptor(kg, b)
-                for q in range(4):
-                    e(f"buffer_store_dword {self.vr('Sum')}, {self.vr('Eff', q)}, {self.sr('RsrcY', 4)}, 0 offen sc0 sc1")
+        e(f"s_cbranch_scc1 {bad_done}")
+        e(f"s_mov_b32 {self.sr('Bad')}, 1")
         e(f"s_branch {bad_done}")
-        self.filters_are_zero(zero, zero_done)
         self.outofline.extend(self.lines)
         self.lines = main
 
     def store_rows(self, kg, out, plain, stored):
-        """The 16 outputs of filter group kg: published past the caches (Kind bit 0), or final ones."""
+        """The 16 outputs of filter group kg: published past the caches as they are (Kind bit 0), or final ones."""
         for policy in (" sc0 sc1", " nt"):
             if policy == " nt":
                 self.label(plain)
@@ -731,6 +727,8 @@ class KernelSplit(Kernel):
             for b in range(4):
                 self.row_descriptor(kg, b)
                 for q in range(4):
+                    if policy == " nt":
+                        self.e(f"v_mul_f32 {out(q, b)}, 0x{UNSCALE:x}, {out(q, b)}")
                     self.e(f"buffer_store_dword {out(q, b)}, {self.vr('Eff', q)}, {self.sr('RsrcY', 4)}, 0 offen{policy}")
             if policy != " nt":
                 self.e(f"s_branch {stored}")
@@ -763,50 +761,6 @@ class KernelSplit(Kernel):
             self.store_rows(kg, out, self.newlabel("store"), self.newlabel("stored"))
         e(f"s_branch {done}")
 
-    def filters_are_zero(self, entry, done):
-        """Sums of zero with inputs that are not: fine when the wave's eight filters are zero (or do not
-        exist), else M = all lanes.  Lane (pp, h, f) reads the two channels of two positions of filter f of a row
-        group: two loads per four channels."""
-        t, e = self.t, self.e
-        loop = self.newlabel("zeroloop")
-        r = lambda i, n=1: v(self.V["EX"] + 48 + i, n)  # no store reads these
-        self.label(entry)
-        e(f"s_lshl_b32 {t(0)}, {self.sr('DkbM')}, 6")
-        e(f"s_lshl_b32 {t(1)}, {self.sr('Wave')}, 2")
-        e(f"s_add_u32 {t(0)}, {t(0)}, {t(1)}")
-        e(f"s_cmp_lt_u32 {t(0)}, {self.sr('Kreal')}")
-        e(f"s_cbranch_scc0 {done}")
-        e(f"v_lshrrev_b32 {r(0)}, 7, {self.vr('Lane16')}")
-        e(f"v_lshlrev_b32 {r(0)}, 10, {r(0)}")                   # pp * 1024
-        e(f"v_lshlrev_b32 {r(1)}, 3, {self.vr('Lane16')}")
-        e(f"v_and_b32 {r(1)}, 0x200, {r(1)}")                    # h * 512
-        e(f"v_and_b32 {r(2)}, 0x30, {self.vr('Lane16')}")
-        e(f"v_add3_u32 {r(0)}, {r(0)}, {r(1)}, {r(2)}")
-        e(f"s_lshl_b32 {t(1)}, {t(1)}, 4")                       # the row group's first filter
-        e(f"v_add_u32 {r(0)}, {t(1)}, {r(0)}")
-        e(f"v_mov_b32 {r(1)}, 0")
-        e(f"s_lshl_b32 {t(0)}, {self.sr('DkbM')}, 1")
-        e(f"s_mul_i32 {t(0)}, {t(0)}, {self.sr('Q')}")
-        e(f"s_add_u32 {t(1)}, {t(0)}, {self.sr('Q')}")
-        e(f"s_lshl_b32 {t(0)}, {t(0)}, 13")
-        e(f"s_lshl_b32 {t(1)}, {t(1)}, 13")
-        e(f"s_mov_b32 {t(4)}, {self.sr('Q')}")
-        self.label(loop)
-        e(f"buffer_load_dwordx4 {r(4, 4)}, {r(0)}, {self.sr('RsrcU', 4)}, {t(0)} offen")
-        e(f"buffer_load_dwordx4 {r(8, 4)}, {r(0)}, {self.sr('RsrcU', 4)}, {t(1)} offen")
-        e(f"s_add_u32 {t(0)}, {t(0)}, 0x2000")
-        e(f"s_add_u32 {t(1)}, {t(1)}, 0x2000")
-        e("s_waitcnt vmcnt(0)")
-        for i in range(4, 12, 2):
-            e(f"v_or3_b32 {r(1)}, {r(i)}, {r(i + 1)}, {r(1)}")
-        e(f"s_sub_u32 {t(4)}, {t(4)}, 1")
-        e(f"s_cmp_lg_u32 {t(4)}, 0")
-        e(f"s_cbranch_scc1 {loop}")
-        e(f"v_lshlrev_b32 {r(1)}, 1, {r(1)}")
-        e(f"v_cmp_ne_u32 vcc, 0, {r(1)}")
-        e(f"s_or_b64 {self.sr('M', 2)}, {self.sr('M', 2)}, vcc")
-        e(f"s_branch {done}")
-
     def stamp(self):
         """Timeline, as Kernel.stamp; the stamp count lives in a register of its own, and the temporaries in
         the registers that hold nothing between two segments."""
@@ -825,7 +779,7 @@ class KernelSplit(Kernel):
         self.stamp()
         self.start()
         self.lds_addresses()
-        self.prologue()
+        self.prologue(False)
         self.stamp()
         self.segments(False)
         end = self.newlabel("end")
@@ -866,7 +820,7 @@ class KernelSplit(Kernel):
         e(f"s_mov_b32 {self.sr('Cm')}, 0")
         self.start()
         self.lds_addresses()
-        self.prologue()
+        self.prologue(True)
         self.segments(True)
         self.label(end)
         e("s_endpgm")
@@ -935,6 +889,7 @@ class KernelSplit(Kernel):
         e(f"s_lshl_b32 {self.sr('ColStep')}, {self.sr('N')}, 2")
         e(f"s_mul_i32 {self.sr('RowStep')}, {self.sr('ColStep')}, {self.sr('W')}")
         e(f"s_mov_b32 {self.sr('MaskHi')}, 0xffff0000")
+        e(f"s_mov_b32 {self.sr('Scale')}, 0x{SCALE:x}")
         e(f"s_mov_b32 {self.sr('Stamps')}, 0")
         e(f"s_mov_b32 {self.sr('Bad')}, 0")
         e(f"s_mov_b32 {s(S['RsrcX'] + 2)}, {self.sr('HWN4')}")
@@ -969,7 +924,7 @@ class KernelSplit(Kernel):
         e(f"v_xor_b32 {self.vr('LdsWr')}, {t(1)}, {self.vr('LdsWr')}")
         e(f"v_add_u32 {self.vr('LdsWr')}, {t(0)}, {self.vr('LdsWr')}")
 
-    def prologue(self):
+    def prologue(self, exact):
         """Unit 0 into V buffer 0, its filters into U, the patch of unit 1 into P; unit 0's patch lands in
         VR, so that all loads leave together."""
         e = self.e
@@ -988,7 +943,7 @@ class KernelSplit(Kernel):
             e(self.patch_load("P", p))
         e(f"s_mov_b32 {self.sr('G')}, 0")
         e("s_waitcnt vmcnt(20)")
-        column, row = self.transform_items("VR", True)
+        column, row = self.transform_items("VR", exact)
         for item in column + row:
             e(item if isinstance(item, str) else item[2])
         e("s_waitcnt vmcnt(0)")  # the first chunk counts on a queue without surprises
@@ -998,7 +953,6 @@ class KernelSplit(Kernel):
         t, e = self.t, self.e
         seg_loop, regular, epi, done = (self.newlabel(x) for x in ("seg", "regular", "epi", "done"))
         self.label(seg_loop)
-        e(f"v_mov_b32 {self.vr('Nz')}, {self.vr('NzNext')}")
         # P is in this tile, or (tiles of one chunk) in the next one
         e(f"s_cmp_eq_u32 {self.sr('Tm')}, {self.sr('Tp')}")
         e(f"s_cselect_b32 {self.sr('DkbM')}, {self.sr('Dkb')}, {self.sr('DkbPrev')}")

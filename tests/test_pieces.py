@@ -38,8 +38,8 @@ def test_kernel_text(split, kw, ragged, packed):
     assert text.count("v_mfma_f32_32x32x16_bf16") == 4 * 24
     assert text.count("v_mfma_f32_32x32x2_f32") == 2 * 32
     # the counted waits rely on STORES stores per output transform: plain, published, merged, merged and
-    # published, exact (and the NaNs of a part that pieces cannot hold)
-    assert text.count("buffer_store_dword") == 6 * split.STORES
+    # published, exact
+    assert text.count("buffer_store_dword") == 5 * split.STORES
     assert len(re.findall(r"buffer_load_dword v\d+, [^\n]* sc0 sc1", text)) == 32  # a partial tile
     assert all(int(n) <= 63 for n in re.findall(r"vmcnt\((\d+)\)", text))
     assert all(int(n) <= 15 for n in re.findall(r"lgkmcnt\((\d+)\)", text))
@@ -135,8 +135,8 @@ def _tensors(shape, seed):
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape", SHAPES)
 def test_every_scale_of_the_operands(ocn, oracle, torch_gpu, shape):
-    # pieces hold 2^-108 ... 2^127; outside (and where outputs come out tiny or huge) the tiles are computed on the
-    # fp32 MFMA.  Relative to the fp64 direct convolution every scale has fp32's accuracy: C roundings of
+    # Split times 2^16, pieces hold all of fp32 below 2^112; beyond (and where outputs come out huge) the tiles are
+    # computed on the fp32 MFMA.  Relative to the fp64 direct convolution every scale has fp32's accuracy: C roundings of
     # 2^-24 and the transforms' (below 1e-6 at these sizes); 2^-132 leaves 2^-17 of a denormal's bits.
     x, w = _tensors(shape, 5)
     want = oracle.direct_conv_f64(x, w).astype(np.float64)
@@ -151,7 +151,7 @@ def test_every_scale_of_the_operands(ocn, oracle, torch_gpu, shape):
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape", SHAPES)
 def test_operands_below_the_pieces(ocn, oracle, torch_gpu, shape):
-    # Denormal inputs that no bf16 piece holds (the sums on pieces are zero), in all channels, in the first or
+    # Denormal inputs, which bf16 pieces hold only because they are scaled, in all channels, in the first or
     # second half of them only (the other half zero: with a tile cut between workgroups, one part says
     # nothing) or in one image; denormal filters; and zeros, which are exact as they are.
     x, w = _tensors(shape, 6)
@@ -181,6 +181,96 @@ def test_operands_below_the_pieces(ocn, oracle, torch_gpu, shape):
     assert not y[: K // 2].any() and np.isfinite(y).all()
     assert not _run(ocn, torch_gpu, np.zeros_like(x), w).any()
     assert not _run(ocn, torch_gpu, x, np.zeros_like(w)).any()
+
+
+def _per_filter(y, want):
+    """Relative 2-norm error of every filter's outputs."""
+    y, want = (t.reshape(t.shape[0], -1) for t in (y, want))
+    return np.linalg.norm(y - want, axis=1) / np.linalg.norm(want, axis=1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ex,ew", [(60, -120), (100, -130), (-120, 60), (-130, 100)])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_small_operands_times_large_ones(ocn, oracle, torch_gpu, shape, ex, ew):
+    # Operands of few bits above 2^-133, where bf16 ends, times such large ones that the outputs are ordinary.
+    # Bound: fp32's error (2e-6, as above), and what the two halvings of the filter transform round off denormal weights: half
+    # a step of 2^-149 each, against weights of the root mean square below.
+    x, w = _tensors(shape, 8)
+    x, w = np.ldexp(x, ex), np.ldexp(w, ew)
+    print(f"small times large {shape} 2^{ex} 2^{ew}", flush=True)
+    rel = _per_filter(_run(ocn, torch_gpu, x, w).astype(np.float64), oracle.direct_conv_f64(x, w).astype(np.float64))
+    assert rel.max() <= 2e-6 + 2.0 ** -149 / np.sqrt(np.mean(w.astype(np.float64) ** 2)), rel.max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES)
+def test_one_small_filter_among_ordinary_ones(ocn, oracle, torch_gpu, shape):
+    # The other filters' outputs say nothing about a filter of small weights: 2^-112 ... 2^-120 hold fp32's accuracy;
+    # of 2^-136 a weight has 13 bits left, and so have its outputs (below 2^-128, in steps of 2^-149).
+    for ew in (-112, -120, -136):
+        x, w = _tensors(shape, 9)
+        k = shape[4] // 2
+        w[..., k] = np.ldexp(w[..., k], ew)
+        print(f"one small filter {shape} 2^{ew}", flush=True)
+        y, want = _run(ocn, torch_gpu, x, w).astype(np.float64), oracle.direct_conv_f64(x, w).astype(np.float64)
+        rel = _per_filter(y, want)
+        assert np.delete(rel, k).max() <= 2e-6
+        if ew > -130:
+            assert rel[k] <= 2e-6, (ew, rel[k])
+        else:  # halvings of the filter transform and sums: fewer than 16 * C steps of the grid, weighted by inputs below 6
+            assert np.abs(y[k] - want[k]).max() <= 6 * 16 * shape[1] * 2.0 ** -149 and rel[k] <= 0.1, rel[k]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("zero_filters", [False, True])
+@pytest.mark.parametrize("N,C,H,K", [(32, 24, 5, 7), (32, 40, 9, 64), (32, 256, 7, 128)])
+def test_small_inputs_in_one_channel(ocn, oracle, torch_gpu, N, C, H, K, zero_filters):
+    # The only inputs that are not zero are denormals of one channel.  With 7 filters most waves store no output; or
+    # the eight filters whose outputs the wave of the channel computes are zero.
+    for c in (2, C - 1):
+        x, w = _tensors((N, C, H, H, K), 10)
+        z = np.zeros_like(x)
+        z[c] = x[c] * np.float32(1e-41)
+        zero = [k for k in range(K) if k % 32 // 4 == c % 8] if zero_filters else []
+        w[..., zero] = 0
+        print(f"one channel N={N} C={C} H={H} K={K} c={c} {zero_filters}", flush=True)
+        y, want = _run(ocn, torch_gpu, z, w), oracle.direct_conv_f64(z, w)
+        assert not y[zero].any()
+        # one channel: halvings and sums of 16 products, fewer than 64 steps of 2^-149 an output
+        assert np.abs(y.astype(np.float64) - want).max() <= 64 * 2.0 ** -149
+        keep = [k for k in range(K) if k not in zero]
+        assert (y[keep] != 0).mean() > 0.9 * (np.abs(want[keep]) > 2.0 ** -149).mean()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ex,ew", [(92, 0), (95, 0), (109, -100), (113, -113), (-90, 110), (-100, 117), (47, 47)])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_both_sides_of_the_largest_operands(ocn, oracle, torch_gpu, shape, ex, ew):
+    # outputs on both sides of 2^94, inputs and weights on both sides of 2^112
+    x, w = _tensors(shape, 11)
+    print(f"largest operands {shape} 2^{ex} 2^{ew}", flush=True)
+    want = np.ldexp(oracle.direct_conv_f64(x, w).astype(np.float64), ex + ew)
+    rel = _per_filter(_run(ocn, torch_gpu, np.ldexp(x, ex), np.ldexp(w, ew)).astype(np.float64), want)
+    assert rel.max() <= 2e-6, rel.max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sx,sw", [(1e-19, 1e-19), (1e-38, 1.0), (1.0, 1e-38), (1e-41, 1.0)])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_denormal_operands_and_products_keep_their_bits(ocn, oracle, torch_gpu, shape, sx, sw):
+    # fp32's error and, on the grid of denormals, half a step of 2^-149 for the output and for each halving of the
+    # filter transform
+    x, w = _tensors(shape, 12)
+    x, w = (x * np.float64(sx)).astype(np.float32), (w * np.float64(sw)).astype(np.float32)
+    print(f"denormals {shape} {sx} {sw}", flush=True)
+    y, want = _run(ocn, torch_gpu, x, w).astype(np.float64), oracle.direct_conv_f64(x, w).astype(np.float64)
+    assert np.abs(want).max() < 1e-36
+    rms = lambda t: np.sqrt(np.mean(t.astype(np.float64) ** 2))
+    rel = np.linalg.norm(y - want) / np.linalg.norm(want)
+    assert rel <= 2e-6 + 2.0 ** -149 / rms(want) + 2.0 ** -149 / rms(w), rel
+    # (an output nearer to zero than one element's error, C roundings of 2^-24 of the terms, may come out as zero)
+    assert (y[np.abs(want) > shape[1] * 2.0 ** -24 * rms(want) + 2.0 ** -148] != 0).all()
 
 
 @pytest.mark.gpu
