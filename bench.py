@@ -28,10 +28,12 @@ PEAK_F16_MFMA_TFLOPS = 2500.0  # dense fp16 / bf16 matrix peak
 PEAK_HBM_GBS = 8000.0
 
 
-def f32_peak(channels):
-    """Matrix peak of an fp32 layer: from 17 channels on the library multiplies three bf16 pieces an
-    operand, six products for one."""
-    return PEAK_F16_MFMA_TFLOPS / 6.0 if channels > 16 else PEAK_FP32_MFMA_TFLOPS
+def matrix_peak(kernel, channels):
+    """Matrix peak of the kernel that ran a layer (opencnn_last_kernel).  The fp32 assembly kernels multiply
+    three bf16 pieces an operand, six products for one, from 17 channels on."""
+    if "f32" not in kernel:
+        return PEAK_F16_MFMA_TFLOPS
+    return PEAK_F16_MFMA_TFLOPS / 6.0 if "_asm_" in kernel and channels > 16 else PEAK_FP32_MFMA_TFLOPS
 
 
 # name -> (N, C, H=W, K, input range, filter distribution)
@@ -110,7 +112,7 @@ class Layer:
                                      self.H, self.K, warmup=warmup, iters=iters, parts=parts)
 
 
-def from_idle(torch, lay, flops_mfma, peak, idle_s=0.5):
+def from_idle(torch, lay, flops_mfma, idle_s=0.5):
     """The reference's own protocol (src/openCNN_winograd.cu:426-444): one warm-up call, then 100
     back-to-back calls between two events, starting from an idle device - no settle phase.  Once
     for the whole call (filter transform + fused kernel) and, after another idle period, once
@@ -122,7 +124,7 @@ def from_idle(torch, lay, flops_mfma, peak, idle_s=0.5):
     _, main, _ = lay.kernel_times(1, 100, parts=("main",))
     return {"protocol": "0.5 s idle, 1 warm-up call, 100 timed calls (HIP events), as the reference's bench",
             "ms_per_step": total, "ms_fused_kernel": main,
-            "frac": flops_mfma / (main * 1e-3) / 1e12 / peak}
+            "frac": flops_mfma / (main * 1e-3) / 1e12 / matrix_peak(lay.ocn.last_kernel(), lay.C)}
 
 
 def settle(torch, lay, ms):
@@ -402,9 +404,8 @@ def main():
     reduced = args.operands != "f32"
     if reduced:
         ocn.set_operand_precision(ocn.F16 if args.operands == "f16" else ocn.BF16)
-    peak = PEAK_F16_MFMA_TFLOPS if reduced else f32_peak(layer.C)
 
-    idle = from_idle(torch, layer, fm, peak)  # first: nothing has run on the device yet
+    idle = from_idle(torch, layer, fm)  # first: nothing has run on the device yet
     settle(torch, layer, args.settle_ms)
     for _ in range(args.warmup):
         layer.step()
@@ -421,6 +422,7 @@ def main():
     achieved = fm / (ms_main * 1e-3) / 1e12
     traffic, traffic_commit = measured_traffic(layer.name + ("_" + args.operands if reduced else ""))
     kernel_name = ocn.last_kernel()
+    peak = matrix_peak(kernel_name, layer.C)
     grid, flag_set = ocn.last_launch()
     ocn.set_operand_precision(ocn.F32)
     ocn.check_status()  # raises if any launch so far gave up a hand-over between workgroups
@@ -497,17 +499,18 @@ def main():
         for name in LAYERS:
             lay = layer if name == layer.name else Layer(ocn, torch, name)
             d, m, b = work(lay.N, lay.C, lay.H, lay.K)
-            precisions = [("f32", ocn.F32, f32_peak(lay.C))]
+            precisions = [("f32", ocn.F32)]
             if name.startswith("reduced"):
-                precisions = [("f16", ocn.F16, PEAK_F16_MFMA_TFLOPS), ("bf16", ocn.BF16, PEAK_F16_MFMA_TFLOPS)]
-            for label, prec, peak in precisions:
+                precisions = [("f16", ocn.F16), ("bf16", ocn.BF16)]
+            for label, prec in precisions:
                 try:
                     ocn.set_operand_precision(prec)
                     settle(torch, lay, args.settle_ms / 2)
                     tot, mn, fx = lay.kernel_times(20, 200)
+                    row_peak = matrix_peak(ocn.last_kernel(), lay.C)
                     # the reference's own protocol on this layer, after the sustained figures: the
                     # idle period it starts with puts the device back into its idle state
-                    idle_row = from_idle(torch, lay, m, peak)
+                    idle_row = from_idle(torch, lay, m)
                 finally:
                     ocn.set_operand_precision(ocn.F32)
                 extra = {}
@@ -519,7 +522,7 @@ def main():
                     "ms_filter_transform": fx,
                     "effective_tflops": d / (tot * 1e-3) / 1e12,
                     "mfma_tflops": m / (mn * 1e-3) / 1e12,
-                    "mfma_frac_of_peak": m / (mn * 1e-3) / 1e12 / peak,
+                    "mfma_frac_of_peak": m / (mn * 1e-3) / 1e12 / row_peak,
                     "from_idle_ms_per_layer": idle_row["ms_per_step"],
                     "from_idle_ms_fused_kernel": idle_row["ms_fused_kernel"],
                     "from_idle_frac": idle_row["frac"],

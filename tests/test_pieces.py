@@ -103,6 +103,16 @@ def test_waits_of_a_chunk_cover_its_loads(split):
             assert not regs & busy, (line, sorted(regs & busy))
 
 
+@pytest.mark.parametrize("kernel,channels,peak", [
+    ("wino_f32_asm_kw2", 64, 2500.0 / 6), ("wino_f32_asm_kw4_packed", 17, 2500.0 / 6), ("wino_f32_asm_kw2", 16, 157.3),
+    ("wino_f32_fused", 64, 157.3), ("wino_f32_fused_lds", 64, 157.3), ("wino_bf16_asm_kw4", 64, 2500.0),
+    ("wino_h16_fused_lds", 16, 2500.0)])
+def test_bench_prices_a_layer_against_the_kernel_that_ran(kernel, channels, peak):
+    import bench  # (a layer of 32 filters may run the register kernel, whatever its channels)
+
+    assert bench.matrix_peak(kernel, channels) == peak
+
+
 # ---------------------------------------------------------------- GPU
 # (N, C, H, W, K): three units with a ragged last one, an odd number of column groups, packed columns, tiles cut
 # between two workgroups, tiles cut among several, two filter blocks with a pair that is not full, a single group
