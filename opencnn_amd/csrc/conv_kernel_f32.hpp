@@ -369,10 +369,14 @@ __global__ void __launch_bounds__(256) wino_f32_fused(ConvArgs a) {
 // its partial result and raises a flag, the second adds its own on top.  a+b == b+a in fp32,
 // so the result does not depend on the arrival order.  The second wave only ever waits for a
 // wave that is already running its epilogue, never for one that has yet to be scheduled.
-constexpr int kMaxBalancedBlocks = 512;
+//
 // [set][boundary between workgroups b and b+1][wave] -> {ticket, flag}; zero between launches
-// (the second contributor clears its pair).  Launches that may overlap in time must not share a
+// (the second contributor clears its pair).  Workgroups of these kernels have four waves, those of the
+// fp32 assembly kernels on pieces eight (their index is boundary * 8 + wave): a set holds eight per
+// boundary, and 512 boundaries (one persistent workgroup per compute unit, 256 on MI355X) keep it at 32 KB,
+// the size that callers who bring flag storage of their own have always been told.  Launches that may overlap in time must not share a
 // set: the host hands one to every stream that launches and to every stream capture (api.hip).
+constexpr int kMaxBalancedBlocks = 512;
 constexpr int kEagerSets = 32;  // streams that launch directly
 constexpr int kGraphSets = 16;  // launches recorded into HIP graphs
 constexpr int kSyncSets = kEagerSets + kGraphSets;

@@ -103,6 +103,99 @@ def test_waits_of_a_chunk_cover_its_loads(split):
             assert not regs & busy, (line, sorted(regs & busy))
 
 
+class Replay:
+    """The counted waits of a whole kernel, on every path through its text: a register that a load or an LDS read is
+    still on its way to must not be read or written.  A state is (line, global accesses in flight, LDS accesses in
+    flight, what is known of Kind); accesses of a kind return in order, so vmcnt(n) leaves the n youngest."""
+
+    def __init__(self, kernel):
+        kernel.body()
+        self.kind = kernel.sr("Kind")
+        self.lines = [l.split(";")[0].strip() for l in kernel.lines]
+        self.labels = {l[:-1]: i for i, l in enumerate(self.lines) if l.endswith(":")}
+
+    @staticmethod
+    def vgprs(text):
+        regs = set()
+        for first, last in re.findall(r"\bv\[(\d+):(\d+)\]", text):
+            regs.update(range(int(first), int(last) + 1))
+        regs.update(int(r) for r in re.findall(r"\bv(\d+)\b", text))
+        return frozenset(regs)
+
+    def run(self):
+        """(line number, line, registers) of the first access that comes too early, or None."""
+        parsed = []
+        for l in self.lines:
+            op, _, rest = l.partition(" ")
+            vm, lds = op.startswith(("buffer_", "global_")), op.startswith("ds_")
+            load = "_load_" in op or op.startswith("ds_read")
+            dst = self.vgprs(rest.split(",")[0]) if load else frozenset()
+            n = {c: int(x) for c, x in re.findall(r"(vmcnt|lgkmcnt)\((\d+)\)", rest)} if op == "s_waitcnt" else {}
+            smem = op.startswith(("s_load", "s_memrealtime"))
+            parsed.append((op, rest, vm, lds or smem, dst, n, self.vgprs(rest)))
+        seen, todo = set(), [(0, (), (), ())]
+        while todo:
+            at, vm, lds, known = state = todo.pop()
+            if state in seen:
+                continue
+            seen.add(state)
+            op, rest, is_vm, is_lds, dst, n, regs = parsed[at]
+            if op == "s_endpgm":
+                continue
+            for q in vm + lds:
+                if q & regs:
+                    return at, self.lines[at], sorted(q & regs)
+            if is_vm:
+                vm += (dst,)
+            elif is_lds:
+                lds += (dst,)
+            if "vmcnt" in n:
+                vm = vm[max(0, len(vm) - n["vmcnt"]):]
+            if "lgkmcnt" in n:
+                lds = lds[max(0, len(lds) - n["lgkmcnt"]):]
+            if op.startswith("s_or_b32") and rest.startswith(self.kind + ","):
+                known = ()
+            if op.startswith("s_cbranch"):
+                taken, passed = (self.labels[rest], vm, lds, known), (at + 1, vm, lds, known)
+                m = re.match(r"s_bitcmp1_b32 (\w+), (\d)", self.lines[at - 1])
+                if m and m.group(1) == self.kind:
+                    bit, on = int(m.group(2)), op == "s_cbranch_scc1"
+                    for value in (dict(known)[bit],) if bit in dict(known) else (True, False):
+                        target = taken if value == on else passed
+                        todo.append(target[:3] + (tuple(sorted({**dict(known), bit: value}.items())),))
+                else:
+                    todo += [taken, passed]
+            elif op == "s_branch":
+                todo.append((self.labels[rest], vm, lds, known))
+            else:
+                todo.append((at + 1, vm, lds, known))
+        return None
+
+
+@pytest.mark.parametrize("ragged,packed", VARIANTS)
+@pytest.mark.parametrize("kw", [2, 4])
+def test_waits_of_a_whole_kernel_cover_its_loads(split, kw, ragged, packed):
+    """Prologue, chunks of every place in a segment, output transforms with and without hand-overs, the exact pass."""
+    assert Replay(split.KernelSplit(kw, ragged, packed)).run() is None
+
+
+def test_replay_of_the_waits_finds_a_wait_that_is_missing(split):
+    """Every counted wait taken out in turn: the replay has to object, except for two waits of each of the four chunks
+    that others cover: that for the patch (its last loads are read behind the wait for U1, the others arrived with U0) and
+    that for the last V reads (they precede the barrier, which waits for all)."""
+    replay = Replay(split.KernelSplit(2))
+    lines = replay.lines
+    waits = [i for i, l in enumerate(lines) if re.match(r"s_waitcnt (vmcnt|lgkmcnt)\([1-9]\d*\)$", l)]
+    assert len(waits) == 36
+    missed = []
+    for i in waits:
+        good, lines[i] = lines[i], ""
+        if replay.run() is None:
+            missed.append(good)
+        lines[i] = good
+    assert len(missed) == 8 and set(missed) == {"s_waitcnt vmcnt(2)", "s_waitcnt vmcnt(34)", "s_waitcnt lgkmcnt(8)"}, missed
+
+
 @pytest.mark.parametrize("kernel,channels,peak", [
     ("wino_f32_asm_kw2", 64, 2500.0 / 6), ("wino_f32_asm_kw4_packed", 17, 2500.0 / 6), ("wino_f32_asm_kw2", 16, 157.3),
     ("wino_f32_fused", 64, 157.3), ("wino_f32_fused_lds", 64, 157.3), ("wino_bf16_asm_kw4", 64, 2500.0),
@@ -121,16 +214,17 @@ SHAPES = [(32, 17, 6, 6, 64), (32, 24, 5, 5, 100), (5, 33, 9, 9, 40), (64, 64, 4
           (33, 40, 12, 13, 300), (16, 136, 9, 9, 32), (3, 20, 14, 11, 7)]
 
 
-def _run(ocn, torch, x, w):
+def _run(ocn, torch, x, w, family="_asm_", **settings):
     C, H, W, N = x.shape
     K = w.shape[3]
     dev = torch.device("cuda:0")
     guard = 1024
     raw = torch.full((K * H * W * N + 2 * guard,), float("nan"), device=dev)
     ws = torch.empty(ocn.workspace_bytes(C, K) // 4, device=dev)
-    ocn.conv_forward_desc(torch.from_numpy(x).to(dev), torch.from_numpy(w).to(dev), raw[guard:-guard], ws, N, C, H, W, K)
+    ocn.conv_forward_desc(torch.from_numpy(x).to(dev), torch.from_numpy(w).to(dev), raw[guard:-guard], ws, N, C, H, W, K,
+                          **settings)
     torch.cuda.synchronize()
-    assert "_asm_" in ocn.last_kernel()
+    assert family in ocn.last_kernel()
     assert torch.isnan(raw[:guard]).all() and torch.isnan(raw[-guard:]).all(), "wrote outside the output"
     return raw[guard:-guard].cpu().numpy().reshape(K, H, W, N)
 
@@ -181,16 +275,32 @@ def test_operands_below_the_pieces(ocn, oracle, torch_gpu, shape):
         if name == "one image":  # the others have fp32's errors at their own scale
             y, direct = y[..., N // 2], direct[..., N // 2]
         # multiples of 2^-149: every halving of a transform and every sum rounds to that grid, fewer than 16 * C
-        # of them an output.  (An output within those steps of zero may come out as zero, hence no count of
-        # them; lost operands would leave no output at all.)
+        # of them an output, most of them far less.  An output of a step or two may come out as zero.
         assert np.abs(y.astype(np.float64) - direct).max() <= 16 * C * 2.0 ** -149
-        assert (y != 0).mean() > 0.5
+        assert (y != 0).mean() >= 0.999 * (np.abs(direct) > 4 * 2.0 ** -149).mean() > 0.9
     zero = w.copy()
     zero[..., : K // 2] = 0
     y = _run(ocn, torch_gpu, x, zero)
     assert not y[: K // 2].any() and np.isfinite(y).all()
     assert not _run(ocn, torch_gpu, np.zeros_like(x), w).any()
     assert not _run(ocn, torch_gpu, x, np.zeros_like(w)).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,pieces", [(s, True) for s in SHAPES] + [((32, 16, 6, 6, 64), False), ((33, 9, 9, 9, 300), False),
+                                                                       ((128, 24, 28, 28, 32), False)])
+def test_which_layers_run_on_pieces(ocn, torch_gpu, shape, pieces):
+    # Both families of fp32 kernels go by the same names.  One channel, one pixel an image and the filters' centre alone:
+    # an output is a single product.  The fp32 MFMA rounds it once; six products of pieces, added up, miss that in some
+    # of the elements, by a step or two.
+    N, C, H, W, K = shape
+    rng = np.random.default_rng(13)
+    x, w = np.zeros((C, H, W, N), np.float32), np.zeros((C, 3, 3, K), np.float32)
+    x[C - 1, 2, 3], w[C - 1, 1, 1] = rng.normal(size=N), rng.normal(size=K)
+    y = _run(ocn, torch_gpu, x, w, family="_asm_" if pieces or K > 32 else "wino_f32_fused")
+    once = w[C - 1, 1, 1][:, None] * x[C - 1, 2, 3][None]
+    steps = np.abs(y[:, 2, 3] - once) / np.spacing(np.abs(once))
+    assert steps.max() <= 2 and (steps != 0).any() == pieces, (steps.max(), (steps != 0).mean())
 
 
 def _per_filter(y, want):
@@ -287,16 +397,17 @@ def test_denormal_operands_and_products_keep_their_bits(ocn, oracle, torch_gpu, 
 @pytest.mark.parametrize("shape", SHAPES)
 def test_non_finite_operands_stay_in_their_tiles(ocn, oracle, torch_gpu, shape):
     # An infinity in the last channel: the same non-finite elements as on the fp32 MFMA everywhere (the
-    # restatement of the reference's arithmetic), finite ones as accurate as ever.
+    # restatement of the reference's arithmetic, or, since that takes square images only, the HIP kernels, which the
+    # restatement checks on square ones), finite ones as accurate as ever.
     N, C, H, W, K = shape
-    if H != W:
-        pytest.skip("the restatement takes square images")
     x, w = _tensors(shape, 7)
     x[C - 1, H // 2, 1, N - 1] = np.inf
     x[0, 0, 0, 0] = np.nan
     print(f"non-finite {shape}", flush=True)
-    y, want = _run(ocn, torch_gpu, x, w), oracle.winograd_f32(x, w)
-    assert np.array_equal(np.isnan(y), np.isnan(want)) and np.array_equal(np.isposinf(y), np.isposinf(want))
-    ok = np.isfinite(want)
-    rel, _, _ = oracle.compare(np.where(ok, y, 0.0), np.where(ok, want, 0.0))
-    assert rel <= 2e-6, rel
+    y, hip = _run(ocn, torch_gpu, x, w), _run(ocn, torch_gpu, x, w, family="wino_f32_", variant=ocn.KERNEL_HIP)
+    for want in [hip] + ([oracle.winograd_f32(x, w)] if H == W else []):
+        assert np.isnan(want).any() and np.array_equal(np.isnan(y), np.isnan(want))
+        assert np.array_equal(np.isposinf(y), np.isposinf(want)) and np.array_equal(np.isneginf(y), np.isneginf(want))
+        ok = np.isfinite(want)
+        rel, _, _ = oracle.compare(np.where(ok, y, 0.0), np.where(ok, want, 0.0))
+        assert rel <= 2e-6, rel
