@@ -509,7 +509,8 @@ int launch_h16(opencnn::ConvArgs a, int precision, hipStream_t st, LaunchPlan* p
 // workgroup whose range ends inside a tile adds, in its output transform, the partial tile that
 // the workgroup behind it published, and publishes the sum if its range also started inside
 // that tile; the workgroup with the tile's first units stores the tile: per tile a chain of
-// hand-overs of about 4 us each, in a fixed order.  Ranges of at least kMinUnitsPerRange units.
+// hand-overs of about 4 us each (fp32 on pieces: 2.5), in a fixed order.  Ranges of at least kMinUnitsPerRange
+// units, fitted to units of 2.2 us and to those of the fp16 / bf16 kernels; not swept on pieces (1.2 us).
 constexpr int kMinUnitsPerRange = 8;
 
 // How a kernel family can cut the tiles of such a layer.
@@ -533,7 +534,9 @@ int pieces_per_tile(int nblocks, int chunks, int cus) {
 int ranges_for_few_tiles(int nblocks, int chunks, int cus) {
   const long long total = (long long)nblocks * chunks;
   // A tile of `chunks` units cut into p ranges takes chunks / p units and p - 1 hand-overs of
-  // about two units each: shortest near p = sqrt(chunks / 2), i.e. ranges of sqrt(2 * chunks) units.
+  // about two units each (2.5 us and 1.2 us on pieces, the only fp32 kernel whose tiles have so many units;
+  // 4 and 2.2 on the fp32 MFMA, where the rule comes from): shortest near p = sqrt(chunks / 2), i.e.
+  // ranges of sqrt(2 * chunks) units.
   int min_units = kMinUnitsPerRange;
   while (min_units * min_units < 2 * chunks) ++min_units;
   long long grid = total / min_units;
@@ -738,9 +741,11 @@ int pack_columns(opencnn::ConvArgs* a, int cw, int kblocks, int chunks, CutTiles
 // 0 = equal numbers of units) lets the slowest range end first.  A range costs its units, and in tenths of a
 // unit: so much per tile it touches (output transform, restart of the pipeline), when it starts inside a tile
 // (that part is published through memory) and when it ends inside one (it waits for the published part).
-// On the fp32 MFMA: fitted to the kernels' times on twelve layers under every weight; the choice it makes
-// there is never slower than the equal split and up to 6.7 % faster (tiles of 8 units, 1.5 - 2.3 tiles per
-// range).  On pieces the units are shorter and the output transform longer: fitted to ten layers under the
+// On the fp32 MFMA: fitted to the kernels' times on twelve layers, tiles of 8 units and more among them, which run
+// on pieces now.  On the tiles of one or two units that are left, every weight is within 4 % of every other, and the
+// choice within 1.6 % of the best (us, equal / chosen / best: N=64 C=3 224x224 K=64 221.0 / 221.0 / 220.9, N=64 C=16
+// 112x112 K=64 84.8 / 83.9 / 82.6, N=100 C=8 30x30 K=100 26.3 / 26.4 / 26.3, N=33 C=12 60x60 K=200 97.3 / 97.1 / 97.1).
+// On pieces the units are shorter and the output transform longer: fitted to ten layers under the
 // weights 0 ... 6, within 1 % of the best weight on all of them but one (with the other kernel's costs up to
 // 5.4 % off: N=96 C=K=256 14x14 75.2 us at weight 0, 70.7 at 5; N=32 C=K=64 56x56 32.1 at 2, 30.8 at 6).
 // Cached per thread: a network has a handful of distinct lines.
@@ -799,8 +804,8 @@ int choose_range_weight(int tiles, int chunks, int ranges, bool pieces) {
 // times the matrix rate and the vector work next to it, but an output transform twice as long: its
 // workgroup exchanges 256 KB through LDS) from three 8-channel units per tile on.  Measured, fused
 // kernel in us, fp32 MFMA / pieces: C = 3, 64 x 224 x 224, K = 64 222 / 231; C = 16, 64 x 112 x 112, K = 64
-// 83.3 / 85.7; C = 24, 64 x 56 x 56, K = 96 58.0 / 54.0; C = 32, 32 x 28 x 28, K = 64 12.4 / 11.0; C = 64,
-// 64 x 56 x 56, K = 64 65.2 / 59.0; C = 512, 128 x 7 x 7, K = 512 128 / 103.
+// 84.2 / 88.8; C = 24, 64 x 56 x 56, K = 96 57.9 / 54.3; C = 32, 32 x 28 x 28, K = 64 12.6 / 10.9; C = 64,
+// 64 x 56 x 56, K = 64 64.4 / 59.7; C = 512, 128 x 7 x 7, K = 512 127 / 105.
 bool split_into_pieces(int chunks) { return chunks >= 3; }
 
 int launch_asm(const opencnn::ConvArgs& a, int kw, int grid, bool ragged, bool packed, size_t lds_bytes,
@@ -1165,9 +1170,9 @@ int launch_on_flag_set(opencnn::ConvArgs& a, const CallSettings& c, LaunchPlan* 
     // row masks of the _ragged kernels).  So: the kw that leaves the fewest such waves, 4 on a tie.
     // A single filter group idles half of the tile: the register variant below is faster (measured, K = 32)
     // unless its workgroups of 128 columns leave half of the compute units without work, which it cannot
-    // cut.  Fused kernel in us, register variant / pieces: its workgroups 196: N=32 C=64 56x56 26.7 / 29.7,
-    // N=128 C=128 28x28 48.4 / 49.4; 98: N=64 C=20 28x28 13.0 / 10.1; 49: N=128 C=64 14x14 22.5 / 15.8; 21:
-    // N=16 C=512 18x18 162 / 31.5.
+    // cut.  Fused kernel in us, register variant / pieces: its workgroups 196: N=32 C=64 56x56 26.4 / 28.9,
+    // N=128 C=128 28x28 46.7 / 46.8; 98: N=64 C=20 28x28 13.0 / 10.2; 49: N=128 C=64 14x14 22.6 / 15.6; 11:
+    // N=16 C=512 18x18 162 / 31.7.
     int kw = (a.kgroups + 3) / 4 * 4 <= (a.kgroups + 1) / 2 * 2 ? 4 : 2;
     if (a.kgroups == 1) {
       int cus = 0;

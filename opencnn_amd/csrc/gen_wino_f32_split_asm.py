@@ -19,21 +19,22 @@ Range: bf16 has no exponents below fp32's, so the pieces of a value below 2^-110
 bf16's grid, 2^-133.  Every operand is therefore split times 2^16: fp32's own grid, 2^-149, then lies on
 bf16's, and the pieces are exact for every value up to 2^112.  The outputs are stored times 2^-32.  V gets
 its factor in the input transform (six instructions a patch), U in front of its split (one a value):
-14 of 241 vector instructions a unit, 0.7 ... 2.4 % of a call (N=1 C=K=64 14x14 19.7 -> 20.2 us,
-N=128 C=K=512 7x7 106.6 -> 107.4).  Deciding by the magnitude of operands or outputs instead where the pieces would lose
+14 of 241 vector instructions a unit, 0.4 ... 2.4 % of a call (N=1 C=K=64 14x14 19.7 -> 20.2 us,
+N=128 C=K=512 7x7 106.0 -> 106.5).  Deciding by the magnitude of operands or outputs instead where the pieces would lose
 bits takes both operands' largest and smallest values, of all waves; an output's neighbours do not tell.
 
 What the pieces cannot hold: infinities and NaNs (their residual is NaN), operands of 2^112 or more and
 outputs of 2^94 or more (infinite once scaled).  A lane therefore sums the magnitudes of the outputs it stores;
 where a sum is not finite, or close to it, the workgroup computes the tiles that it stores once more with
 v_mfma_f32_32x32x2_f32 (exact_chunk), which is what gen_wino_f32_asm.py's kernels always use, and
-stores them again.
+stores them again: a launch then takes 2 to 5 times as long (one NaN, fused kernel: N=128 C=K=128 28x28 98 -> 244 us,
+N=128 C=K=512 7x7 106 -> 252, N=32 C=K=512 7x7 38 -> 183, whose tiles the second pass does not cut).
 
-What bounds it: power on layers that fill the chip (N=128 C=K=512 7x7 runs at 2.03 GHz, the fp32 MFMA
+What bounds it: power on layers that fill the chip (N=128 C=K=512 7x7 runs at 2.07 GHz, the fp32 MFMA
 kernel at 2.49; with every wait taken out it takes as long, at a lower clock), issue on small ones (two
-waves per SIMD, some 360 instructions a unit each; without its MFMAs a unit takes 96 % of the time).
-Fused kernel on the fp32 MFMA / here, us: N=64 C=K=64 56x56 65 / 55, N=128 C=K=128 28x28 110 / 94,
-C=K=256 14x14 106 / 92, C=K=512 7x7 128 / 106, N=1 C=K=64 14x14 22.3 / 17.1.
+waves per SIMD, some 370 instructions a unit each; without its MFMAs a unit takes 96 % of the time).
+Fused kernel on the fp32 MFMA / here, us: N=64 C=K=64 56x56 64.4 / 59.7, N=128 C=K=128 28x28 110 / 97,
+C=K=256 14x14 106 / 95, C=K=512 7x7 127 / 105, N=1 C=K=64 14x14 22.5 / 17.8.
 
 Workgroup: eight waves, one tile of 64 filters x 64 columns (2 x 2 MFMA tiles) for all 16 positions.
 Wave w holds positions 2w and 2w + 1: every U and every V element is read, and split, by one wave of
