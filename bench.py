@@ -30,7 +30,8 @@ PEAK_HBM_GBS = 8000.0
 
 def matrix_peak(kernel, channels):
     """Matrix peak of the kernel that ran a layer (opencnn_last_kernel).  The fp32 assembly kernels multiply
-    three bf16 pieces an operand, six products for one, from 17 channels on."""
+    three bf16 pieces an operand, six products for one, from 17 channels on (but for some packed layers of batches
+    below 11 and at most 40 channels, which have no symbol of their own and are priced with the rest)."""
     if "f32" not in kernel:
         return PEAK_F16_MFMA_TFLOPS
     return PEAK_F16_MFMA_TFLOPS / 6.0 if "_asm_" in kernel and channels > 16 else PEAK_FP32_MFMA_TFLOPS

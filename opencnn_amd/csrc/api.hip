@@ -757,12 +757,13 @@ constexpr RangeCosts kRangeCosts[2] = {{13, 10, 6, 4}, {22, 4, 6, 6}};  // fp32 
 int choose_range_weight(int tiles, int chunks, int ranges, bool pieces) {
   const RangeCosts& costs = kRangeCosts[pieces];
   struct Entry {
-    int tiles, chunks, ranges, weight;  // (the chunks say which kernel)
+    int tiles, chunks, ranges, weight;
+    bool pieces;
   };
   thread_local Entry cache[16] = {};
   thread_local unsigned next = 0;
   for (const Entry& e : cache)
-    if (e.tiles == tiles && e.chunks == chunks && e.ranges == ranges) return e.weight;
+    if (e.tiles == tiles && e.chunks == chunks && e.ranges == ranges && e.pieces == pieces) return e.weight;
   // (a weight has to promise half a percent to replace the equal split, and more than a smaller weight)
   long long best_cost = 0;
   int best = 0;
@@ -796,7 +797,7 @@ int choose_range_weight(int tiles, int chunks, int ranges, bool pieces) {
       best_cost = slowest;
     }
   }
-  cache[next++ % 16] = Entry{tiles, chunks, ranges, best};
+  cache[next++ % 16] = Entry{tiles, chunks, ranges, best, pieces};
   return best;
 }
 
@@ -808,14 +809,25 @@ int choose_range_weight(int tiles, int chunks, int ranges, bool pieces) {
 // 64 x 56 x 56, K = 64 64.4 / 59.7; C = 512, 128 x 7 x 7, K = 512 127 / 105.
 bool split_into_pieces(int chunks) { return chunks >= 3; }
 
-int launch_asm(const opencnn::ConvArgs& a, int kw, int grid, bool ragged, bool packed, size_t lds_bytes,
+// But not packed columns of batches of at most ten images (no multiple of four), at most five units a tile and at most one
+// tile for every second compute unit, where filter blocks come in pairs: a lane's column is (spatial tile, image), so
+// quads of lanes straddle tiles and their patch loads cost up to four times as many address cycles, which few
+// units of few tiles cannot hide.  The tile on pieces gathers every patch once per 64 filters, that on the fp32 MFMA once
+// per 128.  Fused kernel in us, fp32 MFMA / pieces: three units, N=1 50x50 K=69 11.5 / 13.4, N=2 27x27 K=250 11.5 / 13.3;
+// four, N=3 25x64 K=233 13.4 / 14.4; five, N=1 71x83 K=125 15.6 / 16.5; 181 such layers, 0.85 ... 0.97 of the time on
+// pieces.  Outside: six and seven units 0.98 ... 1.02 (11 layers); batch 4 and 8 1.14 ... 1.16 (4); more tiles, up to two a
+// compute unit, 0.83 ... 1.21 (113).
+bool packed_pairs_on_fp32(const opencnn::ConvArgs& a, int kw, int chunks, bool packed, int cus) {
+  return packed && kw == 4 && chunks < 6 && a.N <= 10 && a.N % 4 != 0 && a.nblocks <= cus / 2;
+}
+
+int launch_asm(const opencnn::ConvArgs& a, int kw, bool pieces, int grid, bool ragged, bool packed, size_t lds_bytes,
                hipStream_t st, LaunchPlan* plan) {
   DeviceState* ak = nullptr;
   if (int e = device_state(&ak)) return e;
   AsmLaunch l;
   const int form = packed ? 2 : (ragged ? 1 : 0);
   l.chunks = (a.C + 7) / 8;
-  const bool pieces = split_into_pieces(l.chunks);
   l.fn = ak->f32[pieces][kw == 4][form];
   l.name = kF32Kernels[kw == 4][form];
   l.packed = packed;
@@ -1184,7 +1196,8 @@ int launch_on_flag_set(opencnn::ConvArgs& a, const CallSettings& c, LaunchPlan* 
     opencnn::ConvArgs b = a;
     bool packed = false;
     const int chunks = (b.C + 7) / 8;
-    if (kw > 1 && split_into_pieces(chunks)) {
+    bool pieces = kw > 1 && split_into_pieces(chunks);
+    if (pieces) {
       // workgroup tiles of 64 filters x 2 column tiles; kw = 4: the filter blocks come in pairs
       const int kblocks = (b.kgroups + kw - 1) / kw * (kw / 2);
       if (int e = pack_columns(&b, 2, kblocks, chunks, kCutRanges, &packed)) return e;
@@ -1192,14 +1205,19 @@ int launch_on_flag_set(opencnn::ConvArgs& a, const CallSettings& c, LaunchPlan* 
       REQUIRE(nblocks <= kMaxElems / 8);
       b.nblocks = (int)nblocks;
       b.colblocks = (int)colblocks;
-    } else {
+      int cus = 0;
+      if (int e = compute_units(&cus)) return e;
+      pieces = !packed_pairs_on_fp32(b, kw, chunks, packed, cus);
+    }
+    if (!pieces) {
+      b = a;
       if (int e = pack_columns(&b, 4 / kw, (b.kgroups + kw - 1) / kw, chunks, kCutRanges, &packed)) return e;
       REQUIRE(tile_with(b, kw));
     }
     int grid = 0;
     if (int e = asm_grid(b, kw, chunks, kCutRanges, &grid)) return e;
     if (grid > 0)
-      return launch_asm(b, kw, grid, ragged || b.kgroups % kw != 0, packed, lds_bytes(kw), st, plan);
+      return launch_asm(b, kw, pieces, grid, ragged || b.kgroups % kw != 0, packed, lds_bytes(kw), st, plan);
     REQUIRE(variant != OPENCNN_KERNEL_ASM);
   }
   // The HIP C++ kernels: as many sharing waves as the (rounded-up) filter groups fill whole

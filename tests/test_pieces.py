@@ -286,9 +286,16 @@ def test_operands_below_the_pieces(ocn, oracle, torch_gpu, shape):
     assert not _run(ocn, torch_gpu, x, np.zeros_like(w)).any()
 
 
+# packed columns, pairs of filter blocks: batches up to ten that break quads of lanes, few channels and few tiles keep
+# the fp32 MFMA; an edge of each
+PACKED = [((2, 24, 27, 27, 250), False), ((1, 40, 42, 33, 100), False), ((10, 33, 31, 33, 100), False),
+          ((2, 41, 27, 27, 250), True), ((4, 24, 27, 27, 250), True), ((11, 24, 31, 41, 100), True), ((2, 24, 27, 27, 60), True),
+          ((7, 24, 40, 41, 250), True)]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape,pieces", [(s, True) for s in SHAPES] + [((32, 16, 6, 6, 64), False), ((33, 9, 9, 9, 300), False),
-                                                                       ((128, 24, 28, 28, 32), False)])
+                                                                       ((128, 24, 28, 28, 32), False)] + PACKED)
 def test_which_layers_run_on_pieces(ocn, torch_gpu, shape, pieces):
     # Both families of fp32 kernels go by the same names.  One channel, one pixel an image and the filters' centre alone:
     # an output is a single product.  The fp32 MFMA rounds it once; six products of pieces, added up, miss that in some
@@ -297,7 +304,8 @@ def test_which_layers_run_on_pieces(ocn, torch_gpu, shape, pieces):
     rng = np.random.default_rng(13)
     x, w = np.zeros((C, H, W, N), np.float32), np.zeros((C, 3, 3, K), np.float32)
     x[C - 1, 2, 3], w[C - 1, 1, 1] = rng.normal(size=N), rng.normal(size=K)
-    y = _run(ocn, torch_gpu, x, w, family="_asm_" if pieces or K > 32 else "wino_f32_fused")
+    family = "_kw4_packed" if (shape, pieces) in PACKED and K > 64 else "_asm_" if pieces or K > 32 else "wino_f32_fused"
+    y = _run(ocn, torch_gpu, x, w, family=family)
     once = w[C - 1, 1, 1][:, None] * x[C - 1, 2, 3][None]
     steps = np.abs(y[:, 2, 3] - once) / np.spacing(np.abs(once))
     assert steps.max() <= 2 and (steps != 0).any() == pieces, (steps.max(), (steps != 0).mean())
