@@ -79,3 +79,30 @@ def test_values_that_are_not_finite_stay_in_their_windows(ocn, torch_gpu, N, C, 
     touched[:, 4:8, 4:8, N // 2] = True  # patch rows 2t-1 ... 2t+2 hold row 5 for t = 2, 3; columns 6 the same
     assert np.array_equal(y[~touched], want[~touched])
     assert not np.isfinite(y[:, 5, 6, N // 2]).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,H,W,shallow", [(32, 1831, 1832, True), (32, 1832, 1832, False), (33, 1803, 1804, True), (33, 1804, 1804, False)])
+def test_store_offsets_at_their_limit(ocn, torch_gpu, N, H, W, shallow):
+    # a lane's store offset spans five images: up to 2^31 bytes this kernel, beyond the general one, with every output written
+    print(f"shallow limit N={N} H={H} W={W}", flush=True)
+    torch = torch_gpu
+    C, K = 1, 5
+    assert (20 * N * H * W < 2 ** 31) == shallow
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(7)
+    x = torch.rand(C * H * W * N, device="cuda:0", generator=gen)
+    w = torch.rand(C * 9 * K, device="cuda:0", generator=gen)
+    ws = torch.empty(ocn.workspace_bytes(C, K) // 4, device="cuda:0")
+    y = torch.full((K * H * W * N,), float("nan"), device="cuda:0")
+    ocn.conv_forward_desc(x, w, y, ws, N, C, H, W, K)
+    torch.cuda.synchronize()
+    kernel = ocn.last_kernel()
+    general = torch.full_like(y, float("nan"))
+    ocn.conv_forward_desc(x, w, general, ws, N, C, H, W, K, variant=ocn.KERNEL_REGISTER)
+    torch.cuda.synchronize()
+    assert not torch.isnan(general).any(), "an output element was never written"
+    unwritten = int(torch.isnan(y).sum())
+    assert unwritten == 0, unwritten
+    assert torch.equal(y, general)
+    assert (kernel == "wino_f32_shallow") == shallow
