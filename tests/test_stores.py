@@ -53,3 +53,29 @@ def test_layers_with_cached_stores(ocn, torch_gpu, shape, operands):
     y = runs[0][1024:-1024].view(K, H, W, N).double()
     rel = float((y - want).norm() / want.norm())
     assert rel <= BOUNDS[operands], rel
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("operands", ["F16", "BF16"])
+@pytest.mark.parametrize("H,W,packed", [(1803, 1804, True), (1804, 1804, False)])
+def test_packed_store_offsets_at_their_limit(ocn, torch_gpu, H, W, packed, operands):
+    # on packed columns a lane's store offset spans five images: beyond 2^31 bytes the columns stay unpacked
+    print(f"packed limit H={H} W={W} {operands}", flush=True)
+    torch = torch_gpu
+    N, C, K = 33, 1, 5
+    assert (20 * N * H * W < 2 ** 31) == packed
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(8)
+    x = torch.rand((C, H, W, N), device="cuda:0", generator=gen)
+    w = torch.rand((C, 3, 3, K), device="cuda:0", generator=gen)
+    ws = torch.empty(ocn.workspace_bytes(C, K) // 4, device="cuda:0")
+    y = torch.full((K, H, W, N), float("nan"), device="cuda:0")
+    ocn.conv_forward_desc(x, w, y, ws, N, C, H, W, K, precision=getattr(ocn, operands))
+    torch.cuda.synchronize()
+    unwritten = int(torch.isnan(y).sum())
+    assert unwritten == 0, unwritten
+    # the last rows of every filter, where the offsets are largest
+    want = _exact(torch, x[:, -17:], w)[:, 1:]
+    rel = (y[:, -16:].double() - want).flatten(1).norm(dim=1) / want.flatten(1).norm(dim=1)
+    assert float(rel.max()) <= BOUNDS[operands], rel
+    assert "_asm_" in ocn.last_kernel() and ocn.last_kernel().endswith("_packed") == packed
