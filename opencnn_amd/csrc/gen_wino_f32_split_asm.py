@@ -978,10 +978,14 @@ class KernelSplit(Kernel):
         for item in self.patch_items("P"):
             e(item[2])
         e(f"s_mov_b32 {self.sr('G')}, 0")
+        self.behind_first_loads(exact)
         e(f"s_waitcnt vmcnt({4 + len(first)})")
         self.first_transform(exact)
         e("s_waitcnt vmcnt(0)")  # the first chunk counts on a queue without surprises
         self.swap_buffers()
+
+    def behind_first_loads(self, exact):
+        pass
 
     def first_transform(self, exact):
         column, row = self.transform_items("VR", exact)

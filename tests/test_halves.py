@@ -211,3 +211,30 @@ def test_errors_are_no_larger_than_on_pieces(ocn, oracle, torch_gpu, channels):
     rel = np.linalg.norm(y - want) / np.linalg.norm(want)
     print(f"C={channels} rel {rel:.3e}", flush=True)
     assert rel <= 1.05 * {48: 2.0e-7, 49: 2.0e-7, 64: 2.1e-7, 512: 2.9e-7}[channels]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(64, 64, 40, 40, 64), (32, 256, 7, 7, 128), (33, 56, 42, 41, 100), (1, 64, 14, 14, 64)])
+def test_what_lds_held_before_does_not_matter(ocn, torch_gpu, shape):
+    """A transpose in front of the layer leaves the compute units' LDS full of small integers, like the marks of units out of
+    range: the layer's bits are the same after each of them."""
+    torch = torch_gpu
+    N, C, H, W, K = shape
+    x, w = (torch.from_numpy(t).to("cuda:0") for t in _tensors(shape, 45))
+    x += 0.5  # (every unit is in range)
+    ws = torch.empty(ocn.workspace_bytes(C, K) // 4, device="cuda:0")
+    ocn.filter_transform(w, ws, K, C, ocn.FILTER_CRSK, ocn.WW_MFMA)
+    src = torch.empty(128 * 300000, dtype=torch.int32, device="cuda:0")
+    dst = torch.empty_like(src)
+    outputs = []
+    for mark in [-1, *range(8), 0x7FA00000]:
+        print(f"LDS of {mark} {shape}", flush=True)
+        src.fill_(mark)
+        y = torch.full((K * H * W * N,), float("nan"), device="cuda:0")
+        ocn.nchw_to_chwn(src.view(torch.float32), dst.view(torch.float32), 128, 300000, 1, 1)
+        ocn.conv_forward_desc(x, None, y, ws, N, C, H, W, K)
+        torch.cuda.synchronize()
+        assert bool((dst == mark).all())
+        outputs.append(y)
+    assert not torch.isnan(outputs[0]).any()
+    assert [torch.equal(outputs[0], y) for y in outputs] == [True] * len(outputs)
