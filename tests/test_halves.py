@@ -75,6 +75,93 @@ def test_registers_that_live_through_a_chunk(half, name, offsets, first, last, s
             assert not live & set(range(int(m.group(2)), int(m.group(3) or m.group(2)) + 1)), line
 
 
+def _simulate(items, regs, scalars):
+    """The vector instructions of the range check on 64 lanes; returns vcc."""
+    from test_pieces import Replay
+
+    masks = {}
+    for line in items:
+        if line.startswith("s_nop"):
+            continue
+        op, rest = line.split(" ", 1)
+        args = [a.strip() for a in rest.split(",")]
+
+        def value(a):
+            name = a.strip("|")
+            x = regs[int(name[1:])] if name.startswith("v") else np.full(64, scalars[name] if name in scalars else int(name, 0) & 0xffffffff)
+            return x & 0x7fffffff if a.startswith("|") else x
+        if op.startswith("v_permlane"):
+            a, b = (regs[int(x[1:])].reshape(-1, 32 if "lane32" in op else 16) for x in args)
+            odd = a[1::2].copy()
+            a[1::2], b[0::2] = b[0::2].copy(), odd
+            continue  # (both are views of the registers)
+        if op == "s_or_b64":
+            masks["vcc"] = masks[args[1]] | masks[args[2]]
+            continue
+        src = [value(a).astype(np.uint32) for a in args[1:]]
+        if op.startswith("v_cmp"):
+            x, y = (z.view(np.float32) if op.endswith("f32") else z for z in src)
+            masks[args[0]] = x > y if "_gt_" in op else x < y
+            continue
+        assert args[0] not in ("v0",) and Replay.vgprs(args[0])
+        if op == "v_add_u32":
+            out = src[0] + src[1]
+        else:  # (magnitudes compare as integers do)
+            out = (np.maximum if op.startswith("v_max") else np.minimum).reduce(src)
+        regs[int(args[0][1:])] = out.astype(np.uint32)
+    return masks["vcc"]
+
+
+@pytest.mark.parametrize("name", CLASSES)
+def test_patches_out_of_range(half, name):
+    """The check that units carry against its definition: a patch is out of range if it has a magnitude above V_HIGH, or one of its
+    four 3 x 3 windows (of an output each) has something in it but nothing of V_LOW or more."""
+    k = getattr(half, name)(4, True, True)
+    items = sum(k.magnitude_items("P"), []) + k.patch_range_items(1)[:3]
+    low, high = np.float32(half.V_LOW), np.float32(half.V_HIGH)
+    edges = np.array([0, -0.0, low, np.nextafter(low, np.float32(0)), 1e-45, high, np.nextafter(high, np.float32(100)), 1], np.float32)
+    rng = np.random.default_rng(41)
+    seen = set()
+    for run in range(200):
+        d = np.where(rng.random((64, 4, 4)) < rng.choice([0.3, 0.8, 0.97]), 0, rng.choice(edges, (64, 4, 4))).astype(np.float32)
+        if run % 2:  # in range
+            d = np.where(d > high, high, np.where(d < low, 0, d))
+        d *= rng.choice([-1, 1], d.shape)
+        m = np.abs(d)
+        windows = np.array([m[:, i:i + 3, j:j + 3].max((1, 2)) for i in (0, 1) for j in (0, 1)])
+        want = (m.max((1, 2)) > high) | ((windows > 0) & (windows < low)).any(0)
+        regs = {i: np.zeros(64, np.uint32) for i in range(128)}
+        raw = d.view(np.uint32)
+        for r in range(4):
+            for c in range(4):
+                if name == "KernelHalf":  # a lane's own patch
+                    regs[k.V["P"] + 4 * r + c] = raw[:, r, c].copy()
+                else:  # lane 16 j + q: column j of the patches of columns 4 q + c
+                    regs[k.V["P"] + 4 * r + c] = np.array([raw[4 * (l % 16) + c, r, l // 16] for l in range(64)])
+        got = _simulate(items, regs, {k.sr("VHigh"): int(high.view(np.uint32))})
+        if name == "KernelQuads":  # (each lane tells of another patch than its own)
+            perm = np.array([4 * (l % 16) + (0, 2, 1, 3)[l // 16] for l in range(64)])
+            assert np.array_equal(got, want[perm])
+        else:
+            assert np.array_equal(got, want)
+        seen |= set(want)
+    assert seen == {False, True}
+
+
+def test_rows_and_columns_that_no_output_sees(half):
+    """Behind the last output row or column of an odd size, a patch's last row / column repeats its first one."""
+    k = half.KernelHalf(4, True, True)
+    k.patch_offsets()
+    moves = [re.match(r"\s*v_cndmask_b32 v(\d+), v(\d+), v(\d+), vcc", l) for l in k.lines]
+    first = k.V["VOFF"]
+    moves = [(int(m[1]) - first, int(m[3]) - first) for m in moves if m and m[1] == m[2] and 0 <= int(m[1]) - first < 16]
+    assert moves == [(12 + c, c) for c in range(4)] + [(4 * r + 3, 4 * r) for r in range(4)]
+    k = half.KernelQuads(4, True, True)
+    k.patch_offsets()
+    v = k.V["VOFF"]
+    assert f"v_cndmask_b32 v{v + 3}, v{v + 3}, v{v}, vcc" in k.lines[-1]
+
+
 @pytest.mark.skipif(not os.path.exists(CLANG), reason="ROCm LLVM assembler not installed")
 def test_output_assembles_for_gfx950(tmp_path):
     src = tmp_path / "k.s"
@@ -117,11 +204,11 @@ BOUND = 2e-6
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("ex,ew", [(0, 0), (-7, 0), (-9, 0), (-10, 0), (-11, 0), (-13, 0), (4, 0), (5, 0), (7, 0), (0, -10), (0, -12),
+@pytest.mark.parametrize("ex,ew", [(0, 0), (-7, 0), (-9, 0), (-10, 0), (-11, 0), (-12, 0), (-13, 0), (-14, 0), (2, 0), (3, 0), (4, 0), (5, 0), (7, 0), (0, -10), (0, -12),
                                    (0, -13), (0, -15), (0, 3), (0, 5), (-12, 14), (8, -16)])
 @pytest.mark.parametrize("shape", SHAPES)
 def test_both_sides_of_the_ranges(ocn, oracle, torch_gpu, shape, ex, ew):
-    # patches of 2^-10 ... 63.9 and transformed weights of 2^-17 ... 4: all units in range, some of them, none
+    # windows of 2^-12 ... 15.9 and pairs of transformed weights of 2^-17 ... 4: all units in range, some of them, none
     print(f"range {shape} 2^{ex} 2^{ew}", flush=True)
     x, w = _tensors(shape, 21)
     rel = _per_filter(ocn, oracle, torch_gpu, np.ldexp(x, ex), np.ldexp(w, ew))
@@ -211,6 +298,34 @@ def test_errors_are_no_larger_than_on_pieces(ocn, oracle, torch_gpu, channels):
     rel = np.linalg.norm(y - want) / np.linalg.norm(want)
     print(f"C={channels} rel {rel:.3e}", flush=True)
     assert rel <= 1.05 * {48: 2.0e-7, 49: 2.0e-7, 64: 2.1e-7, 512: 2.9e-7}[channels]
+
+
+# quads of images, whole and ragged, tiles of one segment; packed columns; the kernels for broken quads
+BRIGHT_SHAPES = [(32, 64, 8, 8, 64), (20, 72, 9, 11, 70), (33, 56, 42, 41, 100)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sparse", [False, True])
+@pytest.mark.parametrize("e", [-9, -13, -20, -27, -40, -60])
+@pytest.mark.parametrize("shape", BRIGHT_SHAPES)
+def test_outputs_next_to_a_brighter_region(ocn, oracle, torch_gpu, shape, e, sparse):
+    """Rows, columns and pixels of magnitude 1 on a background of 2^e: an output has fp32's accuracy relative to what its own
+    3 x 3 window holds, also where its tile's patch holds something brighter.  One norm per output pixel."""
+    N, C, H, W, K = shape
+    rng = np.random.default_rng(43)
+    base = rng.uniform(1, 2, size=(C, H, W, N)) * rng.choice([-1, 1], (C, H, W, N))
+    if sparse:  # the background's windows hold one pixel or none
+        base *= rng.random((C, H, W, N)) < 0.1
+    w = _tensors(shape, 44)[1]
+    for where in ((slice(1, 2), slice(None)), (slice(4, 5), slice(None)), (slice(None), slice(3, 4)), (slice(None), slice(6, 7)),
+                  (slice(3, 4), slice(3, 4)), (slice(2, 3), slice(5, 6)), (slice(5, 8), slice(0, 2))):
+        print(f"bright {shape} 2^{e} {sparse} {where}", flush=True)
+        x = np.ldexp(base, e)
+        x[(slice(None), *where)] = rng.normal(size=x[(slice(None), *where)].shape)
+        x = x.astype(np.float32)
+        y, want = _run(ocn, torch_gpu, x, w).astype(np.float64), oracle.direct_conv_f64(x, w).astype(np.float64)
+        error, size = np.sqrt(((y - want) ** 2).sum((0, 3))), np.sqrt((want ** 2).sum((0, 3)))
+        assert (error <= BOUND * size).all(), (error / size).max()
 
 
 @pytest.mark.gpu
