@@ -208,7 +208,7 @@ BOUND = 2e-6
                                    (0, -13), (0, -15), (0, 3), (0, 5), (-12, 14), (8, -16)])
 @pytest.mark.parametrize("shape", SHAPES)
 def test_both_sides_of_the_ranges(ocn, oracle, torch_gpu, shape, ex, ew):
-    # windows of 2^-12 ... 15.9 and pairs of transformed weights of 2^-17 ... 4: all units in range, some of them, none
+    # windows of 2^-12 ... 15.9 and pairs of transformed weights of 2^-14 ... 4: all units in range, some of them, none
     print(f"range {shape} 2^{ex} 2^{ew}", flush=True)
     x, w = _tensors(shape, 21)
     rel = _per_filter(ocn, oracle, torch_gpu, np.ldexp(x, ex), np.ldexp(w, ew))
@@ -353,3 +353,27 @@ def test_what_lds_held_before_does_not_matter(ocn, torch_gpu, shape):
         outputs.append(y)
     assert not torch.isnan(outputs[0]).any()
     assert [torch.equal(outputs[0], y) for y in outputs] == [True] * len(outputs)
+
+
+def _tight(shape, ex, ew, seed):
+    """Inputs and weights of magnitudes 2^e ... 2^(e + 1): all windows on one side of a bound."""
+    N, C, H, W, K = shape
+    rng = np.random.default_rng(seed)
+    draw = lambda e, *size: np.ldexp(rng.uniform(1, 2, size=size) * rng.choice([-1, 1], size), e).astype(np.float32)
+    return draw(ex, C, H, W, N), draw(ew, C, 3, 3, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("channels", [51, 64, 128, 256])
+@pytest.mark.parametrize("ex,ew", [(-10, -3), (-11, -3), (-12, -3), (-13, -3), (2, -3), (3, -3), (4, -3), (-1, -11), (-1, -12), (-1, -13), (-1, -14),
+                                   (-1, -15), (-1, -16), (-1, -17), (-1, 0), (-1, 1), (-1, 2), (-12, -13), (-12, -14), (3, -14)])
+def test_errors_at_the_edges_of_the_ranges(ocn, oracle, torch_gpu, channels, ex, ew):
+    """Just inside and just outside each bound the worst filter errs hardly more than at a scale that no bound comes near
+    (numbers scaled by powers of two err exactly alike in fp32): units that fall to pieces have 1.1 times the halves' error, and
+    near a bound halves lose up to 2^-24 of a window's largest input or a pair's larger weight, next to roundings of 2^-22."""
+    shape = (32, channels, 9, 10, 128)
+    x, w = _tight(shape, 0, 0, 46)
+    middle = _per_filter(ocn, oracle, torch_gpu, np.ldexp(x, -1), np.ldexp(w, -3)).max()
+    edge = _per_filter(ocn, oracle, torch_gpu, np.ldexp(x, ex), np.ldexp(w, ew)).max()
+    print(f"edge C={channels} 2^{ex} 2^{ew}: {edge:.3e}, in the middle {middle:.3e}", flush=True)
+    assert edge <= 1.15 * middle
