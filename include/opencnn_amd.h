@@ -367,9 +367,9 @@ const char *opencnn_last_error(void);
  * Name of the fused kernel that this thread's last successful launch used ("" before the first):
  * a short static string such as "wino_f32_asm_kw2" or "wino_f16_asm_kw4_packed" (the assembly
  * kernels' symbol names; the fp32 ones exist three times under the same names, multiplying bf16 pieces from
- * 17 and fp16 halves from 49 channels on) or "wino_f32_fused_lds" or "wino_f32_shallow" (HIP C++ kernels).  For logs
- * and tests: which
- * kernel family a shape ends up in is the library's choice (see opencnn_set_kernel_variant).
+ * 17 and fp16 halves from 49 channels on) or "wino_f32_fused_lds" or "wino_f32_shallow" (HIP C++ kernels).  For
+ * logs: which kernel a shape ends up in is the library's choice (see opencnn_set_kernel_variant), and
+ * opencnn_last_symbol (opencnn_amd_bench.h) tells the three apart.
  * No counterpart in the reference, whose single kernel is fixed at compile time.
  */
 const char *opencnn_last_kernel(void);

@@ -2,8 +2,8 @@
  * opencnn_amd_bench — bench and test support of libopencnn_amd.so, declared apart from the C ABI a
  * caller of the reference would bind (opencnn_amd.h): the timing loop of the reference's bench,
  * a timeline of the assembly kernels, the order in which they walk through the image, the weight
- * of the ranges of the balanced split, the poll limit of a hand-over, and seeded synthetic
- * tensors.  The settings here (tile order, range weight, timeline buffer, wait limit) belong to
+ * of the ranges of the balanced split, the poll limit of a hand-over, the symbol of the kernel that
+ * ran, and seeded synthetic tensors.  The settings here (tile order, range weight, timeline buffer, wait limit) belong to
  * the CALLING THREAD: they change that thread's later launches and nobody else's.  Results never
  * depend on them (a wait limit small enough to make a hand-over give up excepted, which is what
  * it is for).
@@ -65,6 +65,13 @@ int opencnn_set_wait_limit(unsigned polls);
  * workgroups than it holds records for do not record.  NULL / 0 turns it off (the default).
  */
 int opencnn_set_timeline_buffer(long long *device_buffer, size_t bytes);
+
+/*
+ * Bench and test support: as opencnn_last_kernel, but every kernel has a name of its own.  "fp32:", "pieces:" or
+ * "halves:" (which matrix instructions an fp32 assembly kernel uses: fp32, three bf16 pieces or two fp16 halves an
+ * operand) and the launched symbol with its suffixes, for example "halves:wino_f32_asm_kw2_packed_odd_cached".
+ */
+const char *opencnn_last_symbol(void);
 
 /* Layout of a synthetic input written by opencnn_synth_input. */
 enum { OPENCNN_INPUT_CHWN = 0, OPENCNN_INPUT_NCHW = 1 };

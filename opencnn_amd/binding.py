@@ -74,6 +74,7 @@ EXPORTED_SYMBOLS = {
     ),
     "opencnn_last_error": (ctypes.c_char_p, []),
     "opencnn_last_kernel": (ctypes.c_char_p, []),
+    "opencnn_last_symbol": (ctypes.c_char_p, []),
     "opencnn_last_launch": (_c_int, [ctypes.POINTER(_c_int), ctypes.POINTER(_c_int)]),
     "opencnn_check_status": (_c_int, []),
     "opencnn_release_stream": (_c_int, [_c_void_p]),
@@ -194,6 +195,11 @@ def init() -> None:
 def last_kernel() -> str:
     """Name of the fused kernel this thread's last successful launch used."""
     return lib().opencnn_last_kernel().decode()
+
+
+def last_symbol() -> str:
+    """As last_kernel, with the family of an fp32 assembly kernel ("fp32:", "pieces:", "halves:") and all suffixes of its symbol."""
+    return lib().opencnn_last_symbol().decode()
 
 
 def last_launch():

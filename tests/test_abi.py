@@ -22,7 +22,7 @@ def test_header_symbols_exported(ocn):
     # bench and test support lives in its own header, and only there
     assert set(bench) == {"opencnn_time_forward", "opencnn_set_tile_order", "opencnn_set_range_weight",
                           "opencnn_set_wait_limit", "opencnn_set_timeline_buffer", "opencnn_synth_input",
-                          "opencnn_synth_filter"}
+                          "opencnn_synth_filter", "opencnn_last_symbol"}
     assert not set(api) & set(bench)
     handle = ctypes.CDLL(ocn.LIB_PATH)
     for name in api + bench:

@@ -235,6 +235,7 @@ def test_broken_quads_of_images_with_many_units(ocn, oracle, torch_gpu, shape):
         if image is not None:
             x[..., image] = np.ldexp(x[..., image], -25)
         assert _per_filter(ocn, oracle, torch_gpu, x, w).max() <= BOUND
+        assert "_packed_odd" in ocn.last_symbol()
 
 
 @pytest.mark.gpu
@@ -287,6 +288,29 @@ def test_operands_that_pieces_of_either_scale_lose(ocn, oracle, torch_gpu, shape
         assert _per_filter(ocn, oracle, torch_gpu, x, w).max() <= BOUND
 
 
+# fp32 layers on either side of every line between the assembly kernels
+SYMBOLS = [((32, 16, 14, 14, 64), "fp32:wino_f32_asm_kw2"), ((32, 17, 14, 14, 64), "pieces:wino_f32_asm_kw2_ragged"),
+           ((32, 48, 7, 7, 128), "pieces:wino_f32_asm_kw4"), ((32, 49, 7, 7, 128), "halves:wino_f32_asm_kw4_ragged"),
+           ((32, 56, 7, 7, 128), "halves:wino_f32_asm_kw4"), ((64, 64, 40, 40, 64), "halves:wino_f32_asm_kw2"),
+           # whole quads of images; broken ones below and above twelve units a compute unit
+           ((20, 72, 15, 17, 200), "halves:wino_f32_asm_kw4_packed"), ((16, 136, 9, 9, 32), "halves:wino_f32_asm_kw2_packed"),
+           ((3, 100, 13, 11, 70), "pieces:wino_f32_asm_kw4_packed"), ((33, 128, 14, 14, 128), "pieces:wino_f32_asm_kw4_packed"),
+           ((7, 64, 112, 112, 64), "pieces:wino_f32_asm_kw2_packed_cached"),
+           ((33, 64, 56, 57, 64), "halves:wino_f32_asm_kw2_packed_odd_cached"),
+           ((33, 56, 42, 41, 100), "halves:wino_f32_asm_kw4_packed_odd_cached"), ((17, 472, 28, 28, 64), "halves:wino_f32_asm_kw2_packed_odd"),
+           ((17, 456, 28, 28, 64), "pieces:wino_f32_asm_kw2_packed"),
+           # batches that are not packed need no whole quads
+           ((33, 51, 9, 10, 300), "halves:wino_f32_asm_kw2_ragged"), ((1, 64, 14, 14, 64), "halves:wino_f32_asm_kw2_ragged_cached")]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,symbol", SYMBOLS)
+def test_which_kernel_runs(ocn, torch_gpu, shape, symbol):
+    _run(ocn, torch_gpu, *_tensors(shape, 47))
+    assert ocn.last_symbol() == symbol
+    assert ocn.last_kernel() == symbol.split(":")[1].replace("_odd", "").replace("_cached", "")
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("channels", [48, 49, 64, 512])
 def test_errors_are_no_larger_than_on_pieces(ocn, oracle, torch_gpu, channels):
@@ -295,6 +319,7 @@ def test_errors_are_no_larger_than_on_pieces(ocn, oracle, torch_gpu, channels):
     x, w = _tensors((32, channels, 7, 7, 128), 27)
     want = oracle.direct_conv_f64(x, w).astype(np.float64)
     y = _run(ocn, torch_gpu, x, w).astype(np.float64)
+    assert ocn.last_symbol().startswith("halves:" if channels > 48 else "pieces:")
     rel = np.linalg.norm(y - want) / np.linalg.norm(want)
     print(f"C={channels} rel {rel:.3e}", flush=True)
     assert rel <= 1.05 * {48: 2.0e-7, 49: 2.0e-7, 64: 2.1e-7, 512: 2.9e-7}[channels]

@@ -12,6 +12,11 @@ LAYERS += [((36, 51, 43, 43, 64), "F32"), ((36, 51, 31, 31, 128), "F32"), ((33, 
 LAYERS += [((n, 20, h, w, k), p) for form in (PACKED, RAGGED) for n, h, w, k in form.values() for p in ("F16", "BF16")]
 LAYERS += [((3, 64, 14, 14, 64), "F32"), ((1, 9, 7, 7, 128), "F32"), ((5, 20, 6, 6, 64), "F32"), ((3, 20, 9, 9, 64), "F16")]
 LAYERS += [((12, 9, 74, 74, 64), "F32"), ((12, 9, 73, 74, 64), "F32")]
+# stored past the caches: that last one, batches of whole half lines (one of halves, for pairs), packed batches that divide 32, and
+# small outputs of batches of 8 or more
+PAST_CACHES = [LAYERS[-1], ((48, 9, 40, 41, 64), "F32"), ((80, 64, 25, 26, 100), "F32"), ((8, 64, 93, 93, 64), "F32"), ((9, 64, 14, 14, 64), "F32"),
+               ((48, 20, 40, 41, 64), "F16"), ((8, 20, 93, 93, 64), "BF16")]
+LAYERS += PAST_CACHES[1:]
 # fp32: some twenty roundings of 2^-23 on a path; fp16 / bf16: both operands of a product rounded, 2^-11 / 2^-8 each
 BOUNDS = {"F32": 20 * 2.0 ** -23, "F16": 2 * 2.0 ** -11, "BF16": 2 * 2.0 ** -8}
 
@@ -45,6 +50,7 @@ def test_layers_with_cached_stores(ocn, torch_gpu, shape, operands):
         ocn.conv_forward_desc(x, w, raw[1024:-1024], ws, N, C, H, W, K, precision=getattr(ocn, operands))
         torch.cuda.synchronize()
         assert "_asm_" in ocn.last_kernel()
+        assert ocn.last_symbol().endswith("_cached") == ((shape, operands) not in PAST_CACHES), ocn.last_symbol()
         assert torch.isnan(raw[:1024]).all() and torch.isnan(raw[-1024:]).all(), "wrote outside the output"
         assert not torch.isnan(raw[1024:-1024]).any(), "an output element was never written"
         runs.append(raw.clone())
