@@ -28,13 +28,13 @@ PEAK_F16_MFMA_TFLOPS = 2500.0  # dense fp16 / bf16 matrix peak
 PEAK_HBM_GBS = 8000.0
 
 
-def matrix_peak(kernel, channels):
-    """Matrix peak of the kernel that ran a layer (opencnn_last_kernel).  The fp32 assembly kernels multiply
-    three bf16 pieces an operand, six products for one, from 17 channels on (but for some packed layers of batches
-    below 11 and at most 40 channels, which have no symbol of their own and are priced with the rest)."""
-    if "f32" not in kernel:
+def matrix_peak(symbol):
+    """Matrix peak of the kernel that ran a layer (opencnn_last_symbol).  The fp32 assembly kernels make three products of
+    fp16 halves of one fp32 product, six of bf16 pieces, or one on the fp32 matrix instructions, as the HIP kernels do."""
+    if "f32" not in symbol:
         return PEAK_F16_MFMA_TFLOPS
-    return PEAK_F16_MFMA_TFLOPS / 6.0 if "_asm_" in kernel and channels > 16 else PEAK_FP32_MFMA_TFLOPS
+    products = {"halves": 3.0, "pieces": 6.0}.get(symbol.split(":")[0])
+    return PEAK_F16_MFMA_TFLOPS / products if products else PEAK_FP32_MFMA_TFLOPS
 
 
 # name -> (N, C, H=W, K, input range, filter distribution)
@@ -125,7 +125,7 @@ def from_idle(torch, lay, flops_mfma, idle_s=0.5):
     _, main, _ = lay.kernel_times(1, 100, parts=("main",))
     return {"protocol": "0.5 s idle, 1 warm-up call, 100 timed calls (HIP events), as the reference's bench",
             "ms_per_step": total, "ms_fused_kernel": main,
-            "frac": flops_mfma / (main * 1e-3) / 1e12 / matrix_peak(lay.ocn.last_kernel(), lay.C)}
+            "frac": flops_mfma / (main * 1e-3) / 1e12 / matrix_peak(lay.ocn.last_symbol())}
 
 
 def settle(torch, lay, ms):
@@ -422,8 +422,8 @@ def main():
     _, ms_main, ms_fx = layer.kernel_times(args.warmup, args.steps)
     achieved = fm / (ms_main * 1e-3) / 1e12
     traffic, traffic_commit = measured_traffic(layer.name + ("_" + args.operands if reduced else ""))
-    kernel_name = ocn.last_kernel()
-    peak = matrix_peak(kernel_name, layer.C)
+    kernel_name = ocn.last_symbol()
+    peak = matrix_peak(kernel_name)
     grid, flag_set = ocn.last_launch()
     ocn.set_operand_precision(ocn.F32)
     ocn.check_status()  # raises if any launch so far gave up a hand-over between workgroups
@@ -508,7 +508,7 @@ def main():
                     ocn.set_operand_precision(prec)
                     settle(torch, lay, args.settle_ms / 2)
                     tot, mn, fx = lay.kernel_times(20, 200)
-                    row_peak = matrix_peak(ocn.last_kernel(), lay.C)
+                    row_peak = matrix_peak(ocn.last_symbol())
                     # the reference's own protocol on this layer, after the sustained figures: the
                     # idle period it starts with puts the device back into its idle state
                     idle_row = from_idle(torch, lay, m)

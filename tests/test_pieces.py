@@ -196,14 +196,15 @@ def test_replay_of_the_waits_finds_a_wait_that_is_missing(split):
     assert len(missed) == 8 and set(missed) == {"s_waitcnt vmcnt(2)", "s_waitcnt vmcnt(34)", "s_waitcnt lgkmcnt(8)"}, missed
 
 
-@pytest.mark.parametrize("kernel,channels,peak", [
-    ("wino_f32_asm_kw2", 64, 2500.0 / 6), ("wino_f32_asm_kw4_packed", 17, 2500.0 / 6), ("wino_f32_asm_kw2", 16, 157.3),
-    ("wino_f32_fused", 64, 157.3), ("wino_f32_fused_lds", 64, 157.3), ("wino_bf16_asm_kw4", 64, 2500.0),
-    ("wino_h16_fused_lds", 16, 2500.0)])
-def test_bench_prices_a_layer_against_the_kernel_that_ran(kernel, channels, peak):
-    import bench  # (a layer of 32 filters may run the register kernel, whatever its channels)
+@pytest.mark.parametrize("symbol,peak", [
+    ("halves:wino_f32_asm_kw2", 2500.0 / 3), ("halves:wino_f32_asm_kw4_packed_odd_cached", 2500.0 / 3),
+    ("pieces:wino_f32_asm_kw4_packed", 2500.0 / 6), ("fp32:wino_f32_asm_kw2", 157.3), ("wino_f32_shallow", 157.3),
+    ("wino_f32_fused", 157.3), ("wino_f32_fused_lds", 157.3), ("wino_bf16_asm_kw4", 2500.0), ("wino_f16_asm_kw4_ragged_cached", 2500.0),
+    ("wino_h16_fused_lds", 2500.0)])
+def test_bench_prices_a_layer_against_the_kernel_that_ran(symbol, peak):
+    import bench
 
-    assert bench.matrix_peak(kernel, channels) == peak
+    assert bench.matrix_peak(symbol) == peak
 
 
 # ---------------------------------------------------------------- GPU
