@@ -64,10 +64,13 @@ enum {
  * opencnn_filter_transform(..., OPENCNN_WW_MFMA) and the fused kernel must run under the same
  * setting: the library remembers what it wrote to a Ww address and the fused kernel returns
  * hipErrorInvalidValue for a buffer written under another precision (see opencnn_filter_transform).
- * OPENCNN_F32 has fp32's accuracy for every finite operand, denormal ones too, whatever the kernel.
- * From 17 channels on the time depends on the data in one way: infinities, NaNs, operands of 2^112 or more and outputs
- * of 2^94 or more make the workgroups that meet them compute their tiles a second time, another way (a launch then
- * takes 2 to 5 times as long).
+ * OPENCNN_F32 has fp32's accuracy for every finite operand, denormal ones too, whatever the kernel: relative to the
+ * largest input of an output's own 3x3 window and the largest weight of its filter, channel by channel.
+ * The time depends on the data in two ways.  From 17 channels on infinities, NaNs, operands of 2^112 or more and
+ * outputs of 2^94 or more make the workgroups that meet them compute their tiles a second time, another way (a launch
+ * then takes 2 to 5 times as long).  From 49 channels on groups of 8 channels and 64 columns take 1.5 times as long
+ * where an input is above 63.9, where a 3x3 window is not zero but holds nothing of 2^-11 or more, or where a
+ * filter's transformed weights are above 4 or below 2^-14 (a launch, where that is so everywhere: 1.1 to 1.4 times).
  */
 enum { OPENCNN_F32 = 0, OPENCNN_F16 = 1, OPENCNN_BF16 = 2 };
 int opencnn_set_operand_precision(int precision);
